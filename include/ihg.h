@@ -139,6 +139,14 @@ int ihg_rk4_final(ihg_ctx *c, double *y, const double *k1, const double *k2,
  *     order), sums[1] = sum (yerr/sk)^2 (3rd order).  Synchronises. */
 int ihg_dp853_stage(ihg_ctx *c, int s, double dt, const double *y,
                     const double *const *k, double *out);
+/* ihg_dp853_stage for a caller that takes the stages in order, each followed
+ * by its mk_rhs into k[s - 1]: stage 9 also starts the sums of stages 10 to
+ * 12, in k[9], k[10] and k[11] (which their slopes fill afterwards), and
+ * those stages go on from there.  The stage inputs are ihg_dp853_stage's bit
+ * for bit; 12 of the 72 state vectors that the sums move are saved.  The
+ * arrays of k must be distinct from each other and from y and out. */
+int ihg_dp853_stage_ahead(ihg_ctx *c, int s, double dt, const double *y,
+                          double *const *k, double *out);
 int ihg_dp853_finish(ihg_ctx *c, double dt, const double *y,
                      const double *const *k, double *y_new, double rtol,
                      double atol, double sums[2]);
@@ -196,6 +204,10 @@ int ihg_dp853_dense_tableau(double *c_extra, double *a_extra, double *d);
  *     a[13][12], b[13], w[13] (w = e for err_mode 0, bhat for 1). */
 int ihg_gsl_stage(ihg_ctx *c, int method, int s, double dt, const double *y,
                   const double *const *k, double *out);
+/* as ihg_dp853_stage_ahead (RK8PD: stage 9 starts the sums of stages 10 to
+ * 13 in k[9] .. k[12]; RKF45 and RKCK: ihg_gsl_stage) */
+int ihg_gsl_stage_ahead(ihg_ctx *c, int method, int s, double dt,
+                        const double *y, double *const *k, double *out);
 int ihg_gsl_finish(ihg_ctx *c, int method, double dt, const double *y,
                    const double *const *k, double *y_new, double eps_abs,
                    double eps_rel, double *rmax);

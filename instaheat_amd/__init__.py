@@ -171,10 +171,11 @@ IHG_SYMBOLS = [
     "ihg_stream_copy",
     "ihg_sync", "ihg_fft_r2c", "ihg_fft_c2r", "ihg_set_field", "ihg_mk_rhs",
     "ihg_means", "ihg_observables", "ihg_calls_rhs", "ihg_mk_initial_psi",
-    "ihg_rk4_stage", "ihg_rk4_final", "ihg_dp853_stage", "ihg_dp853_finish",
+    "ihg_rk4_stage", "ihg_rk4_final", "ihg_dp853_stage",
+    "ihg_dp853_stage_ahead", "ihg_dp853_finish",
     "ihg_dp853_finish_noalloc", "ihg_mean", "ihg_variance", "ihg_diff_norms",
     "ihg_dp853_tableau", "ihg_dp853_dense_stage", "ihg_dp853_dense",
-    "ihg_dp853_dense_tableau", "ihg_gsl_stage", "ihg_gsl_finish",
+    "ihg_dp853_dense_tableau", "ihg_gsl_stage", "ihg_gsl_stage_ahead", "ihg_gsl_finish",
     "ihg_gsl_tableau", "ihg_download_strided", "ihg_aux", "ihg_prof_enable", "ihg_prof_reset",
     "ihg_prof_read", "ihg_prof_nfam", "ihg_prof_family", "ihg_features",
     "ihg_set_gw_fp32", "ihg_init_gaussian", "ihg_autotune", "ihg_fft_candidates",
@@ -242,6 +243,7 @@ def lib():
         "ihg_rk4_stage": (i, [_vp, _vp, _vp, _vp, d, i]),
         "ihg_rk4_final": (i, [_vp, _vp, _vp, _vp, _vp, _vp, d]),
         "ihg_dp853_stage": (i, [_vp, i, d, _vp, ctypes.POINTER(_vp), _vp]),
+        "ihg_dp853_stage_ahead": (i, [_vp, i, d, _vp, ctypes.POINTER(_vp), _vp]),
         "ihg_dp853_finish": (i, [_vp, d, _vp, ctypes.POINTER(_vp), _vp, d, d,
                                  _dptr]),
         "ihg_dp853_finish_noalloc": (i, [_vp, ctypes.c_long, ctypes.c_long, d,
@@ -258,6 +260,8 @@ def lib():
         "ihg_download_strided": (i, [_vp, _vp, ctypes.POINTER(ctypes.c_int), _dptr]),
         "ihg_gsl_stage": (i, [_vp, i, i, ctypes.c_double, _vp,
                               ctypes.POINTER(_vp), _vp]),
+        "ihg_gsl_stage_ahead": (i, [_vp, i, i, ctypes.c_double, _vp,
+                                    ctypes.POINTER(_vp), _vp]),
         "ihg_gsl_finish": (i, [_vp, i, ctypes.c_double, _vp, ctypes.POINTER(_vp),
                                _vp, ctypes.c_double, ctypes.c_double, _dptr]),
         "ihg_gsl_tableau": (i, [i, ctypes.POINTER(ctypes.c_int), _dptr, _dptr,

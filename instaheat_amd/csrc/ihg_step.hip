@@ -90,6 +90,76 @@ __global__ __launch_bounds__(RED_WG) void k_dp_stage(
     }
 }
 
+// A stage sum that also starts the sums of the NP stages after it: those
+// stages take the same slopes again (DOPRI853's stages 9 to 12 all use k0,
+// k3 .. k7), so their partial sums p_q = sum_j c_qj k_j are formed while the
+// slopes are in registers, and each later stage reads one partial sum
+// instead of six slopes.  The bound is HBM traffic: 60 state vectors a
+// DOPRI853 step move through the stage sums instead of 72, 67 instead of 83
+// for the 13 stages of RK8PD (a RK8PD step at 128^3 with its two saves 7.25
+// -> 6.83 ms, two DOPRI853 steps at 256^3 90.4 -> 86.0 ms).  The terms of every sum are added in the order
+// of k_dp_stage, so the values are the same bit for bit.
+struct AheadOut {
+    double *p[4];
+    double c[4][12];
+};
+
+template <bool NT, int NP>
+__global__ __launch_bounds__(RED_WG) void k_dp_stage_ahead(
+    double *__restrict__ out, const double *__restrict__ y, StageIn s,
+    AheadOut ah, double dt, long nlive, long Ntot)
+{
+    const long npairs = nlive / 2;
+    const long stride = (long)gridDim.x * RED_WG;
+    const double2 *y2 = reinterpret_cast<const double2 *>(y);
+    double2 *o2 = reinterpret_cast<double2 *>(out);
+    for (long i = (long)blockIdx.x * RED_WG + threadIdx.x; i < npairs;
+         i += stride) {
+        const double2 k0 = ld2<NT>(reinterpret_cast<const double2 *>(s.k[0]) + i);
+        double ax = s.a[0] * k0.x, ay = s.a[0] * k0.y;
+        double px[NP], py[NP];
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            px[q] = ah.c[q][0] * k0.x;
+            py[q] = ah.c[q][0] * k0.y;
+        }
+#pragma unroll
+        for (int j = 1; j < 12; ++j) {
+            if (j < s.nk) {
+                const double2 kj =
+                    ld2<NT>(reinterpret_cast<const double2 *>(s.k[j]) + i);
+                ax += s.a[j] * kj.x;
+                ay += s.a[j] * kj.y;
+#pragma unroll
+                for (int q = 0; q < NP; ++q) {
+                    px[q] += ah.c[q][j] * kj.x;
+                    py[q] += ah.c[q][j] * kj.y;
+                }
+            }
+        }
+        const double2 yy = ld2<NT>(y2 + i);
+        st2<NT>(o2 + i, make_double2(yy.x + dt * ax, yy.y + dt * ay));
+#pragma unroll
+        for (int q = 0; q < NP; ++q)
+            st2<NT>(reinterpret_cast<double2 *>(ah.p[q]) + i,
+                    make_double2(px[q], py[q]));
+    }
+    if (blockIdx.x == 0 && threadIdx.x <= NP) {
+        // the scale factor: thread 0 the stage, thread q the partial q - 1
+        const long i = Ntot - 1;
+        const int q = (int)threadIdx.x - 1;
+        double acc = 0.0;
+        for (int j = 0; j < s.nk; ++j) {
+            const double w = q < 0 ? s.a[j] : ah.c[q][j];
+            acc = j ? acc + w * s.k[j][i] : w * s.k[j][i];
+        }
+        if (q < 0)
+            out[i] = y[i] + dt * acc;
+        else
+            ah.p[q][i] = acc;
+    }
+}
+
 // dense output: out = y + beta (y_new - y) + dt * sum_j w_j k_j, the
 // interpolant of an accepted step at one theta (weights from the host)
 template <bool NT>
@@ -527,6 +597,92 @@ extern "C" int ihg_dp853_stage(ihg_ctx *c, int s, double dt, const double *y,
     });
 }
 
+// Stage `s` of a method of `stages` stages with weight rows A (row s - 1 of
+// stage s, `pitch` apart), its stages taken in order: at stage `at` the sums
+// of the later stages are started, each in the array k[s - 1] that its own
+// slope fills afterwards, and a later stage goes on from there.  k[j] and out
+// must not overlap.
+static int stage_ahead(ihg_ctx *c, int s, int stages, int at, const double *A,
+                       int pitch, double dt, const double *y,
+                       double *const *k, double *out, int fam)
+{
+    const double *row = A + (s - 1) * pitch;
+    StageIn in{};
+    int n = 0;
+    if (s > at) { // the sum of the terms before k[at - 1], started there
+        IHG_TRY(check_ptr(k[s - 1], "k[s - 1]"));
+        in.k[n] = k[s - 1];
+        in.a[n++] = 1.0;
+    }
+    int col[12];
+    for (int j = s > at ? at - 1 : 0; j < s - 1; ++j) {
+        if (row[j] == 0.0) continue;
+        IHG_TRY(check_ptr(k[j], "k[j]"));
+        col[n] = j;
+        in.k[n] = k[j];
+        in.a[n++] = row[j];
+    }
+    in.nk = n;
+    const long nl = live_len(c);
+    const int np = s == at ? stages - at : 0;
+    AheadOut ah{};
+    for (int q = 0; q < np; ++q) {
+        IHG_TRY(check_ptr(k[at + q], "k[later stage]"));
+        ah.p[q] = k[at + q];
+        for (int j = 0; j < n; ++j)
+            ah.c[q][j] = A[(at + q) * pitch + col[j]];
+    }
+    return timed(c, fam, (n + 2.0 + np) * 8.0 * nl, [&]() {
+        const dim3 grid(stream_blocks(nl / 2)), wg(RED_WG);
+        const bool nt = streaming(nl);
+        if (np == 3)
+            hipLaunchKernelGGL((nt ? k_dp_stage_ahead<true, 3>
+                                   : k_dp_stage_ahead<false, 3>),
+                               grid, wg, 0, c->stream, out, y, in, ah, dt, nl,
+                               c->Ntot);
+        else if (np == 4)
+            hipLaunchKernelGGL((nt ? k_dp_stage_ahead<true, 4>
+                                   : k_dp_stage_ahead<false, 4>),
+                               grid, wg, 0, c->stream, out, y, in, ah, dt, nl,
+                               c->Ntot);
+        else
+            hipLaunchKernelGGL((nt ? k_dp_stage<true> : k_dp_stage<false>),
+                               grid, wg, 0, c->stream, out, y, in, dt, nl,
+                               c->Ntot);
+        return hip_check(hipGetLastError(), "k_dp_stage_ahead");
+    });
+}
+
+// The sums of the stages after AHEAD are started at stage AHEAD: every
+// column that a later row has before column AHEAD - 1 must be one that row
+// AHEAD reads, since only those slopes are in registers there.
+template <class Row>
+static constexpr bool ahead_ok(const Row *A, int stages, int at)
+{
+    for (int s = at; s < stages; ++s)
+        for (int j = 0; j < at - 1; ++j)
+            if (A[s][j] != 0.0 && A[at - 1][j] == 0.0) return false;
+    return true;
+}
+
+// Stage 9 of DOPRI853 (stages 8 and 9 move the least: 60 of 72 vectors) and
+// of RK8PD (stage 8: 68, stage 9: 67 of 83).
+constexpr int DP_AHEAD = 9, GSL_AHEAD = 9;
+static_assert(ahead_ok(DP_A, 12, DP_AHEAD), "columns of the later stages");
+static_assert(ahead_ok(GSL_RK8PD.a, 13, GSL_AHEAD), "columns of the later stages");
+
+extern "C" int ihg_dp853_stage_ahead(ihg_ctx *c, int s, double dt,
+                                     const double *y, double *const *k,
+                                     double *out)
+{
+    if (!c || !k) return set_error("NULL argument");
+    if (s < 2 || s > 12) return set_error("stage %d out of range 2..12", s);
+    IHG_TRY(check_ptr(y, "y"));
+    IHG_TRY(check_ptr(out, "out"));
+    return stage_ahead(c, s, 12, DP_AHEAD, &DP_A[0][0], 12, dt, y, k, out,
+                       F_DP_STAGE);
+}
+
 extern "C" int ihg_dp853_dense_stage(ihg_ctx *c, int s, double dt,
                                      const double *y, const double *const *k,
                                      double *out)
@@ -904,6 +1060,24 @@ extern "C" int ihg_gsl_stage(ihg_ctx *c, int method, int s, double dt,
                            c->Ntot);
         return hip_check(hipGetLastError(), "k_dp_stage (gsl)");
     });
+}
+
+extern "C" int ihg_gsl_stage_ahead(ihg_ctx *c, int method, int s, double dt,
+                                   const double *y, double *const *k,
+                                   double *out)
+{
+    const GslTableau *t = gsl_tableau_of(method);
+    if (!c || !k) return set_error("NULL argument");
+    if (!t) return set_error("GSL stepper %d is not 1, 2 or 3", method);
+    if (s < 2 || s > t->stages)
+        return set_error("stage %d out of range 2..%d", s, t->stages);
+    // the five stage sums of the 4(5) pairs have little to share (23 of 25
+    // vectors at best)
+    if (t->stages < 13) return ihg_gsl_stage(c, method, s, dt, y, k, out);
+    IHG_TRY(check_ptr(y, "y"));
+    IHG_TRY(check_ptr(out, "out"));
+    return stage_ahead(c, s, t->stages, GSL_AHEAD, &t->a[0][0],
+                       GSL_MAX_STAGES - 1, dt, y, k, out, F_GSL_STAGE);
 }
 
 // f(std::integral_constant<int, n>) for the weighted-stage counts of the

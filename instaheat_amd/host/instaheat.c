@@ -447,17 +447,17 @@ double ih_error_norm(double e5, double e3, double dt, size_t ntot)
 /* try_step (src/dopri853.c:331-458) + error (:469-486) */
 static int try_step(ih_sim *s, double t, double dt, double *err)
 {
-    const double *k[12];
+    double *k[12];
     k[0] = s->dfield;
     for (int j = 1; j < 12; ++j) k[j] = s->stage[j];
     for (int st = 2; st <= 12; ++st) {
-        int rc = ihg_dp853_stage(s->g, st, dt, s->field, k, s->k_tmp);
+        int rc = ihg_dp853_stage_ahead(s->g, st, dt, s->field, k, s->k_tmp);
         const double ts = (st == 12) ? t + dt : t + s->dp_c[st - 1] * dt;
         if (!rc) rc = ih_mk_rhs(s, ts, s->k_tmp, s->stage[st - 1]);
         if (rc) return rc;
     }
     double sums[2];
-    int rc = ihg_dp853_finish(s->g, dt, s->field, k, s->field_new,
+    int rc = ihg_dp853_finish(s->g, dt, s->field, (const double *const *)k, s->field_new,
                               s->cfg.rtol, s->cfg.atol, sums);
     if (rc) return rc;
     *err = ih_error_norm(sums[0], sums[1], dt, s->Ntot);
@@ -723,7 +723,7 @@ static int gsl_evolve(ih_sim *s, int method, int stages, int order,
 {
     const ih_config *c = &s->cfg;
     const double t0 = s->t, dt = t1 - t0;
-    const double *k[13];
+    double *k[13];
     k[0] = s->dfield;
     for (int j = 1; j < stages; ++j) k[j] = s->stage[j - 1];
     int rc = ih_mk_rhs(s, t0, s->field, s->dfield);
@@ -732,11 +732,11 @@ static int gsl_evolve(ih_sim *s, int method, int stages, int order,
         int final_step = h0 > dt;
         if (final_step) h0 = dt;
         for (int j = 2; j <= stages && !rc; ++j) {
-            rc = ihg_gsl_stage(s->g, method, j, h0, s->field, k, s->k_tmp);
+            rc = ihg_gsl_stage_ahead(s->g, method, j, h0, s->field, k, s->k_tmp);
             if (!rc) rc = ih_mk_rhs(s, t0 + cc[j - 1] * h0, s->k_tmp, s->stage[j - 2]);
         }
         double r = 0.0;
-        if (!rc) rc = ihg_gsl_finish(s->g, method, h0, s->field, k, s->field_new,
+        if (!rc) rc = ihg_gsl_finish(s->g, method, h0, s->field, (const double *const *)k, s->field_new,
                                      c->atol, c->rtol, &r);
         if (rc) return rc;
         ++st->attempts;
