@@ -719,7 +719,7 @@ static int group_rhs(ihg_group *g, double *const *f, double *const *result,
         IHG_TRY(glaunch(g, up, "grouped update_phi_psi"));
     }
 
-    // rhs_gw: z r2c of the six source products, x pass, the fused y pass +
+    // rhs_gw: z r2c of the source products, x pass, the fused y pass +
     // TT projection + update_h (src/toolbox.c:311-424)
     {
         std::vector<Seg<FamSources>> sz;
@@ -736,7 +736,7 @@ static int group_rhs(ihg_group *g, double *const *f, double *const *result,
             s.grid = dim3((unsigned)((nrows + B - 1) / B), 1, nr);
             s.a = {c->grad3, c->W, M, nrows, N, c->tw, e.g, e.w};
             sz.push_back(s);
-            sx.push_back(strided_seg<-1>(c, c->W, x_lines_of(c), 6, M));
+            sx.push_back(strided_seg<-1>(c, c->W, x_lines_of(c), GW_NC, M));
             const LineSet ls = y_lines_of(c);
             const int Bt = dispatch_len(L, [&](auto Lc) {
                 constexpr int LL = decltype(Lc)::value;

@@ -12,7 +12,7 @@
 //                                                         (toolbox.c:140-243)
 //   means           block sums -> rho_mean, pressure_mean, da   (:87, :241)
 //   update          result[0..4N) from f, lap, p, means   (toolbox.c:282-299)
-// GW on adds: z r2c of the six products d_i phi d_j phi (pairs in one complex
+// GW on adds: z r2c of five products of d_i phi d_j phi (pairs in one complex
 // row), an x pass, and one y pass that also does the TT projection and the h
 // update (toolbox.c:311-424).
 #include <cfloat>
@@ -210,7 +210,7 @@ int rhs_core(ihg_ctx *c, double *f, double *result, int output, int kept,
     });
 }
 
-// GW source pipeline on complex type C: z r2c of the six products, x pass,
+// GW source pipeline on complex type C: z r2c of the products, x pass,
 // fused y pass + TT + update_h.  Wk holds 6 M values of C, g3 the gradients;
 // realization r of an ensemble finds them r * rw and r * rg further on.
 template <class C>
@@ -226,7 +226,7 @@ static int rhs_gw_t(ihg_ctx *c, const typename CT<C>::R *g3, C *Wk,
         constexpr int L = decltype(Lc)::value;
         using TL = Tile<L>;
         const unsigned nb = (unsigned)((nrows + TL::B - 1) / TL::B);
-        return timed(c, F_Z_R2C_SRC, (3.0 * rs * N + 6.0 * cs * M) * nr, [&]() {
+        return timed(c, F_Z_R2C_SRC, (3.0 * rs * N + GW_NC * cs * M) * nr, [&]() {
             hipLaunchKernelGGL((k_z_r2c_sources<L, C>), dim3(nb, 1, nr),
                                dim3(FFT_WG), 0, c->stream, g3, Wk, M, nrows, N,
                                tw, rg, rw);
@@ -234,10 +234,10 @@ static int rhs_gw_t(ihg_ctx *c, const typename CT<C>::R *g3, C *Wk,
         });
     }));
     if constexpr (std::is_same<C, float2>::value)
-        IHG_TRY(x_pass_f32(c, Wk, -1, 6, M, nr, rw));
+        IHG_TRY(x_pass_f32(c, Wk, -1, GW_NC, M, nr, rw));
     else
-        IHG_TRY(x_pass(c, Wk, -1, 6, M, nr, rw));
-    // y pass of the six sources, TT projection and update_h: six sources
+        IHG_TRY(x_pass(c, Wk, -1, GW_NC, M, nr, rw));
+    // y pass of the sources, TT projection and update_h: the sources
     // and h1, h2, dh1, dh2 in; the four h blocks of result out
     if constexpr (std::is_same<C, double2>::value) {
         if (ep)
@@ -248,7 +248,7 @@ static int rhs_gw_t(ihg_ctx *c, const typename CT<C>::R *g3, C *Wk,
                 const LineSet ls{(long)c->Nx * c->Mz, c->Mz, (long)c->Ny * c->Mz, c->Mz};
                 const unsigned nb = (unsigned)((ls.nlines + B - 1) / B);
                 const double epb = ep->mode == RK4_FINAL ? 8.0 : 16.0;
-                return timed(c, F_TT_UPDATE_H, (6.0 * 16.0 + (8.0 + epb) * 16.0) * M * nr, [&]() {
+                return timed(c, F_TT_UPDATE_H, (GW_NC * 16.0 + (8.0 + epb) * 16.0) * M * nr, [&]() {
                     hipLaunchKernelGGL((k_y_tt_update_h_rk4<L, TP::WG, typename TP::P>),
                                        dim3(nb, 1, nr), dim3(TP::WG), 0, c->stream, Wk,
                                        M, f, result, N, c->Next, c->Ntot, c->kg,
@@ -266,7 +266,7 @@ static int rhs_gw_t(ihg_ctx *c, const typename CT<C>::R *g3, C *Wk,
         // lines along y: one per (x, kz); points Mz apart
         const LineSet ls{(long)c->Nx * c->Mz, c->Mz, (long)c->Ny * c->Mz, c->Mz};
         const unsigned nb = (unsigned)((ls.nlines + B - 1) / B);
-        return timed(c, F_TT_UPDATE_H, (6.0 * cs + 8.0 * 16.0) * M * nr, [&]() {
+        return timed(c, F_TT_UPDATE_H, (GW_NC * cs + 8.0 * 16.0) * M * nr, [&]() {
             hipLaunchKernelGGL((k_y_tt_update_h<L, TP::WG, typename TP::P, C>),
                                dim3(nb, 1, nr), dim3(TP::WG), 0, c->stream, Wk,
                                M, f, result, N, c->Next, c->Ntot, c->kg,

@@ -304,12 +304,23 @@ __global__ __launch_bounds__(RED_WG) void k_update_phi_psi(
 }
 
 // ---------------------------------------------------------------------------
-// GW sources: z r2c of the six products d_i phi d_j phi (mk_gw_sources,
-// src/toolbox.c:410-424).  A work-group owns B rows: every thread loads its
-// first-stage points of d_x phi, d_y phi, d_z phi once into registers, then
-// the three complex rows (S11, S12), (S13, S22), (S23, S33) of each row are
-// transformed one after the other; component c = 2q + s goes to W + c M.
+// GW sources: z r2c of the products d_i phi d_j phi (mk_gw_sources,
+// src/toolbox.c:410-424).  Only the transverse traceless part of the source
+// enters the equations, and the projection takes delta_ij s to 0 for every s
+// (P is a projector of trace 2 built from the full k with k_i k_i = k^2), so
+// d_z phi d_z phi is subtracted from the diagonal: five components (xx - zz,
+// xy, xz, yy - zz, yz) are transformed instead of six.  That takes a sixth
+// off the transforms of the source (two DOPRI853 steps at 256^3 86.0 -> 83.9
+// ms, 5 RK4 steps of 48 x 32^3 + 16 x 64^3 + 4 x 128^3 50.6 -> 49.0 ms); the
+// error of the slopes of h against 64-bit torch is what it was with six
+// (8e-16 to 1.5e-15 of the source alone, 4^3 to 512-point lines).
+// A work-group owns B rows: every thread loads its first-stage points of
+// d_x phi, d_y phi, d_z phi once into registers, then the complex rows (xx -
+// zz, xy), (xz, yy - zz), (yz, 0) of each row are transformed one after the
+// other; component c = 2q + s goes to W + c M.
 // ---------------------------------------------------------------------------
+constexpr int GW_NC = 5;
+
 template <int L, int Q, class C, class Rows>
 __device__ __forceinline__ void sources_pair(C *lds, int tid, const Rows &g,
                                              bool act, C *__restrict__ W,
@@ -323,23 +334,24 @@ __device__ __forceinline__ void sources_pair(C *lds, int tid, const Rows &g,
     auto rd = [&](int s, int) {
         R u, v;
         if constexpr (Q == 0) {
-            u = g.x[s] * g.x[s];
+            u = g.x[s] * g.x[s] - g.z[s] * g.z[s];
             v = g.x[s] * g.y[s];
         } else if constexpr (Q == 1) {
             u = g.x[s] * g.z[s];
-            v = g.y[s] * g.y[s];
+            v = g.y[s] * g.y[s] - g.z[s] * g.z[s];
         } else {
             u = g.y[s] * g.z[s];
-            v = g.z[s] * g.z[s];
+            v = 0;
         }
         return act ? CT<C>::make(u, v) : CT<C>::make(0, 0);
     };
     fft_line_wave<L, -1, typename TL::P>(lds + bc * TL::PITCH, tid % TL::T, tw, rd);
     // each wavefront splits and stores the rows of its own lines
+    constexpr int NS = Q == 2 ? 1 : 2; // components of the pair
     const int w = tid / 64, lane = tid % 64;
-    for (int idx = lane; idx < TL::LPW * 2 * MZ; idx += 64) {
-        const int lb = w * TL::LPW + idx / (2 * MZ);
-        const int rem = idx - (lb - w * TL::LPW) * 2 * MZ;
+    for (int idx = lane; idx < TL::LPW * NS * MZ; idx += 64) {
+        const int lb = w * TL::LPW + idx / (NS * MZ);
+        const int rem = idx - (lb - w * TL::LPW) * NS * MZ;
         const int s = rem / MZ, k = rem - s * MZ;
         const long r = row0 + lb;
         if (r < nrows)
@@ -396,14 +408,15 @@ __global__ __launch_bounds__(FFT_WG) void k_z_r2c_sources(
 
 // ---------------------------------------------------------------------------
 // TT projection (mk_gw_sources_tt, src/toolbox.c:363-397) as two linear forms
-// of the six source components: o0 = sum_c alpha_c S_c, o1 = sum_c beta_c S_c.
+// of the source components: o0 = sum_c alpha_c S_c, o1 = sum_c beta_c S_c.
 // With f = k / k^2 (full k), t1 = sum_ij k_i f_j S_ij, t2 = tr S, s1 = t1 + t2,
 // s2 = t1 - t2 and the kept axis pair (p, q) = (x, y) if |kz| > eps, (x, z)
 // if |ky| > eps, (y, z) otherwise, the reference computes
 //   o0 = S_pp - 2 f_p (sum_j k_j S_pj) + (f_p k_p s1 + s2) / 2
 //   o1 = S_pq - f_p (sum_j k_j S_qj) - f_q (sum_j k_j S_pj) + f_p k_q s1 / 2
 // alpha_C, beta_C are the derivatives of these with respect to component
-// C = 0..5 = (xx, xy, xz, yy, yz, zz); the k = 0 mode projects to 0.
+// C = 0..4 = (xx, xy, xz, yy, yz) (zz is subtracted from the diagonal); the
+// k = 0 mode projects to 0.
 // ---------------------------------------------------------------------------
 template <int C, class R>
 __device__ __forceinline__ void tt_coef(R kx, R ky, R kz, R inv_ksq,
@@ -429,12 +442,9 @@ __device__ __forceinline__ void tt_coef(R kx, R ky, R kz, R inv_ksq,
     } else if constexpr (C == 3) {
         t1 = ky * fy; t2 = I; rowp = py ? ky : O; rowq = qy ? ky : O;
         dpp = py ? I : O; dpq = O;
-    } else if constexpr (C == 4) {
+    } else {
         t1 = D * (ky * fz); t2 = O; rowp = py ? kz : O;
         rowq = qy ? kz : ky; dpp = O; dpq = py ? I : O;
-    } else {
-        t1 = kz * fz; t2 = I; rowp = O; rowq = qy ? O : kz;
-        dpp = O; dpq = O;
     }
     const R s1 = t1 + t2, s2 = t1 - t2;
     const R half = (R)0.5, two = (R)2.0;
@@ -463,9 +473,9 @@ __device__ __forceinline__ void tt_component(
     // Register pressure control (empty asm statements, no instructions):
     // an opaque zero offset of the twiddle pointer per component (the
     // pointer itself stays visibly an LDS one) stops the compiler from
-    // loading every stage twiddle once and holding it across all six
+    // loading every stage twiddle once and holding it across all the
     // transforms, and pinning the accumulators after each component stops it
-    // from deferring the sums (and so keeping all six spectra live).
+    // from deferring the sums (and so keeping every spectrum live).
     int zo = 0;
     asm volatile("" : "+s"(zo));
     const C *twc = tw + zo;
@@ -476,7 +486,7 @@ __device__ __forceinline__ void tt_component(
     auto acc = [&](int s, int n, C v) {
         // recomputed per component from 1/k^2 alone: an empty asm keeps the
         // compiler from holding every derived coefficient of every point
-        // live across the six transforms
+        // live across the transforms
         R iv = inv_ksq[s];
         asm volatile("" : "+v"(iv));
         const bool zero = z0 && (n == 0);
@@ -518,7 +528,7 @@ __host__ __device__ constexpr int tt_lds()
     return 2 * (WG / (L / P::E)) * Lds<L>::PITCH + L;
 }
 
-// Last pass of the GW sources: y transforms of the six components (z and x
+// Last pass of the GW sources: y transforms of the components (z and x
 // passes done), the TT projection, and update_h (src/toolbox.c:311-346):
 //   dh = hdot,  dhdot = -(2 p_mean + k^2/a^2) h - 3 H hdot + 2 S^TT / a^2
 // (EP: the RK4 epilogue of the four h blocks' slopes)
@@ -613,28 +623,28 @@ __device__ __forceinline__ void y_tt_update_h_body(
     load(1, bufs[1]);
     auto step = [&](auto kc) {
         constexpr int K = decltype(kc)::value;
-        if constexpr (K == 5 && EARLY) load_h();
+        if constexpr (K == GW_NC - 1 && EARLY) load_h();
         tt_component<L, P, K>(K % 2 ? lb1 : lb0, K % 2 ? lw1 : lw0, j, jw, tw,
                               bufs[K % 2], kg, kxw, kzw, b1w, z0w, inv, o0,
                               o1);
-        if constexpr (K + 2 < 6) load(K + 2, bufs[K % 2]);
+        if constexpr (K + 2 < GW_NC) load(K + 2, bufs[K % 2]);
     };
     step(std::integral_constant<int, 0>{});
     step(std::integral_constant<int, 1>{});
     step(std::integral_constant<int, 2>{});
     step(std::integral_constant<int, 3>{});
     step(std::integral_constant<int, 4>{});
-    step(std::integral_constant<int, 5>{});
-    // the two sums back to the load layout through LDS: o0 to buffer 0 (no
-    // wavefront reads it after component 5's barrier), o1 to this
-    // wavefront's own line of buffer 1 once its last reads of it are done
-#pragma unroll
-    for (int s = 0; s < E; ++s)
-        lw0[Lds<L>::idx(last_point<L, P>(jw, s))] = o0[s];
-    line_sync<true>();
+    // the two sums back to the load layout through LDS: o1 to buffer 1 (no
+    // wavefront reads it after the last component's barrier), o0 to this
+    // wavefront's own line of buffer 0 once its last reads of it are done
+    static_assert(GW_NC == 5, "the last component is in buffer 0");
 #pragma unroll
     for (int s = 0; s < E; ++s)
         lw1[Lds<L>::idx(last_point<L, P>(jw, s))] = o1[s];
+    line_sync<true>();
+#pragma unroll
+    for (int s = 0; s < E; ++s)
+        lw0[Lds<L>::idx(last_point<L, P>(jw, s))] = o0[s];
     lds_barrier();
 #pragma unroll
     for (int s = 0; s < E; ++s) {
