@@ -39,8 +39,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, HERE)
 
 METRIC = "sim-time/wall-s at 256³ FP64 DOPRI853 rtol 1e-10: tuned vs plain GPU"
-FFT_FAMILIES = ("z_r2c", "z_c2r", "y_pass", "x_pass", "x_fanout", "z_c2r_rho",
-                "z_r2c_sources", "y_tt_update_h", "x_roundtrip")
+FFT_FAMILIES = ("z_r2c", "z_c2r", "y_pass", "x_pass", "xy_deriv", "z_rhs",
+                "y_tt_update_h", "x_roundtrip")
 # the passes that do nothing but transform (the others fuse derivatives,
 # rho and p, the GW products, the TT projection or the filter into a pass)
 FFT_PLAIN = ("z_r2c", "z_c2r", "y_pass", "x_pass")

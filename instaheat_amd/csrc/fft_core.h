@@ -14,6 +14,13 @@
 
 #include <hip/hip_runtime.h>
 
+// Multiply-adds are fused within an expression only, from here to the end of
+// the unit: which of two products a sum fuses is then fixed by the source.
+// (With fusion across statements the choice depends on the kernel that a
+// body is inlined in, and a grouped launch could differ from the per-context
+// one in the last bit.)
+#pragma clang fp contract(on)
+
 namespace ihg {
 
 // complex value types: double2 (FP64 path) and float2 (the FP32 GW source)
@@ -370,6 +377,15 @@ __device__ __forceinline__ constexpr int chain_slot(int s1)
     return (u % ML) * RL + u / ML;
 }
 
+// and back: the first-stage slot whose point is in last-stage slot `sl`
+template <int L, class P = Plan<L>>
+__device__ __forceinline__ constexpr int unchain_slot(int sl)
+{
+    for (int s = 0; s < P::E; ++s)
+        if (chain_slot<L, P>(s) == sl) return s;
+    return 0;
+}
+
 struct NoRead {
     __device__ double2 operator()(int, int) const { return make_double2(0.0, 0.0); }
 };
@@ -464,6 +480,16 @@ __device__ __forceinline__ void fft_line(C *line, int j,
 {
     fft_line_impl<L, DIR, FIRST_FROM_RD, LAST_TO_WR, P, C, false>(line, line, j,
                                                                   tw, rd, wr);
+}
+
+// A line whose threads are lanes of one wavefront, first stage from `rd`,
+// every output point to `wr` (the caller syncs before the line is reused).
+template <int L, int DIR, class P, class C = double2, class Rd, class Wr>
+__device__ __forceinline__ void fft_line_wave_regs(C *line, int j,
+                                                   const C *__restrict__ tw,
+                                                   Rd rd, Wr wr)
+{
+    fft_line_impl<L, DIR, true, true, P, C, true>(line, line, j, tw, rd, wr);
 }
 
 // A line whose threads are lanes of one wavefront, first stage from `rd`,

@@ -20,12 +20,14 @@ constexpr int FFT_WG = 256;
 
 // Line plans of the z passes.  Their transposes are wavefront-local, so an
 // extra stage costs LDS traffic but no work-group barrier, and fewer values
-// per thread buy occupancy: 256 points take 8 values per thread in three
-// stages (at 16 values the z c2r + rho pass held 182 registers and 70 KB of
-// LDS per work-group, 2 waves per SIMD).  (512 points keep 16 values: a
-// wavefront must hold both lines of a row pair.)
+// per thread buy occupancy: at most 8 values per thread.  The short lines
+// take 2 or 4, so that a small grid spreads over more lanes.
 template <int L> struct ZPlanOf { using P = Plan<L>; };
+template <> struct ZPlanOf<4> { using P = PlanT<2, 2, 2>; };
+template <> struct ZPlanOf<8> { using P = PlanT<4, 4, 2>; };
+template <> struct ZPlanOf<16> { using P = PlanT<4, 4, 4>; };
 template <> struct ZPlanOf<256> { using P = PlanT<8, 8, 8, 4>; };
+template <> struct ZPlanOf<512> { using P = PlanT<8, 8, 8, 8>; };
 
 // Tile of a z pass: B lines of L points per work-group, T threads per line
 template <int L>
@@ -199,84 +201,152 @@ auto with_cand(int id, CandList<C0, Cs...>, F &&f)
 }
 
 // ---------------------------------------------------------------------------
-// x-axis forward transform followed by NQ backward transforms of the same
-// spectrum, each multiplied by its own factor fac(q, line, kx_index, value):
-// the spectral derivatives of the right-hand side (NQ = 4, out of place,
-// output q at out + q * qstride) and the filter round trip (NQ = 1, in
-// place, batched over blockIdx.y with arrays `batch` apart); realizations
-// of an ensemble over blockIdx.z, `rr` apart.
-// The spectrum never leaves registers: the forward transform's last stage
-// keeps its outputs, and each backward transform's first stage takes them
-// through chain_slot; HBM is read once and written NQ times.  With FWD =
-// false the input is already the full spectrum and only the backward
-// transforms run.
+// x-axis forward transform, a factor fac(bk, line, kx_index, value) and the
+// backward transform, in place: the filter round trip, batched over
+// blockIdx.y with arrays `batch` apart, realizations of an ensemble over
+// blockIdx.z, `rr` apart.  The spectrum never leaves registers: the forward
+// transform's last stage keeps its outputs, and the backward transform's
+// first stage takes them through chain_slot; HBM is read and written once.
 // ---------------------------------------------------------------------------
-template <int L, int NQ, bool FWD, class Fac, class P = Plan<L>,
-          int WG = FFT_WG, bool SWZ = true>
-__device__ __forceinline__ void x_fanout_body(
-    const Blk &bk, double2 *lds, const double2 *in, double2 *out,
-    long qstride, LineSet ls, long batch, const double2 *__restrict__ tw,
-    Fac fac, long rr)
+template <int L, class Fac, class P = Plan<L>, int WG = FFT_WG>
+__device__ __forceinline__ void x_roundtrip_body(
+    const Blk &bk, double2 *lds, double2 *data, LineSet ls, long batch,
+    const double2 *__restrict__ tw, Fac fac, long rr)
 {
     constexpr int E = P::E, B = StridedShape<L, P, WG>::B, PITCH = Lds<L>::PITCH;
     const int tid = threadIdx.x;
-    in += bk.y * batch + bk.z * rr;
-    out += bk.y * batch + bk.z * rr;
+    data += bk.y * batch + bk.z * rr;
     const int b = tid % B, j = tid / B;
-    const long line = (long)tile_x<SWZ>(bk) * B + b;
+    const long line = (long)tile_x<true>(bk) * B + b;
     const bool act = line < ls.nlines;
-    const long base = ls.base(act ? line : 0);
-    const double2 *src = in + base;
+    double2 *dst = data + ls.base(act ? line : 0);
     const long st = ls.stride;
     double2 *my = lds + b * PITCH;
     double2 spec[E];
     auto rd = [&](int, int n) {
-        const double2 v = ldn(src + n * st); // in bounds for every lane
+        const double2 v = ldn(dst + n * st); // in bounds for every lane
         return act ? v : make_double2(0.0, 0.0);
     };
-    if constexpr (FWD) {
-        auto keep = [&](int slot, int, double2 v) { spec[slot] = v; };
-        fft_line<L, -1, true, true, P>(my, j, tw, rd, keep);
-    } else {
-#pragma unroll
-        for (int slot = 0; slot < E; ++slot)
-            spec[slot] = rd(slot, stage1_point<L, P>(j, slot));
-    }
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        if (FWD || q > 0)
-            lds_barrier(); // LDS reads of the previous transform are done
-        double2 *dst = out + q * qstride + base;
-        auto rq = [&](int slot, int n) {
-            return fac(bk, q, line, n, spec[FWD ? chain_slot<L, P>(slot) : slot]);
-        };
-        auto wq = [&](int, int n, double2 v) {
-            if (act) stn(dst + n * st, v);
-        };
-        fft_line<L, +1, true, true, P>(my, j, tw, rq, wq);
-    }
+    auto keep = [&](int slot, int, double2 v) { spec[slot] = v; };
+    fft_line<L, -1, true, true, P>(my, j, tw, rd, keep);
+    lds_barrier(); // LDS reads of the forward transform are done
+    auto rq = [&](int slot, int n) {
+        return fac(bk, line, n, spec[chain_slot<L, P>(slot)]);
+    };
+    auto wq = [&](int, int n, double2 v) {
+        if (act) stn(dst + n * st, v);
+    };
+    fft_line<L, +1, true, true, P>(my, j, tw, rq, wq);
 }
 
-template <int L, int NQ, bool FWD, class Fac, class P = Plan<L>,
-          int WG = FFT_WG, bool SWZ = true>
-__global__ __launch_bounds__(WG) void k_x_fanout(
-    const double2 *in, double2 *out, long qstride, LineSet ls, long batch,
-    const double2 *__restrict__ tw, Fac fac, long rr)
+// Work-group size of the round trip per line length.  Measured with 128, 256
+// and 512 lanes: one 32^3 grid 5.1, 5.6, 7.3 us (9 work-groups at 256 leave
+// the chip idle), 64^3 11.3, 11.5, 12.2, 128^3 38.8, 39.3, 55.5, 256^3 423,
+// 343, 348 (128-byte runs at 128 lanes).
+template <int L> struct RoundtripWG { static constexpr int WG = L <= 64 ? 128 : 256; };
+
+template <int L, class Fac, class P = Plan<L>, int WG = FFT_WG>
+__global__ __launch_bounds__(WG) void k_x_roundtrip(
+    double2 *data, LineSet ls, long batch, const double2 *__restrict__ tw,
+    Fac fac, long rr)
 {
     __shared__ double2 lds[StridedShape<L, P, WG>::LDS];
-    x_fanout_body<L, NQ, FWD, Fac, P, WG, SWZ>(hw_blk(), lds, in, out, qstride,
-                                               ls, batch, tw, fac, rr);
+    x_roundtrip_body<L, Fac, P, WG>(hw_blk(), lds, data, ls, batch, tw, fac, rr);
 }
 
-// Line plans of the derivative fan-out.  (At 256 points, 8 values per
-// thread in three stages -- PlanT<8, 8, 8, 4>, 166 VGPRs and 3 waves per
-// SIMD instead of 1 -- measured 209-219 us against 190-194 us for the
-// two-stage 16-value plan, with the XCD-aware tile order on both, and
-// still 198-210 against 172-180 us with the stage twiddles read from LDS
-// (158 VGPRs); the 16-value plan loads its twiddles once for all five
-// transforms, so LDS twiddles gain it nothing either (181-184 us).  The
-// default plans stay.)
-template <int L> struct FanPlan { using P = Plan<L>; static constexpr int WG = FFT_WG; };
+// ---------------------------------------------------------------------------
+// Spectral derivatives along x or y: of every line of the real field phi the
+// forward transform, times i k / L and -k^2 / L, and two backward transforms
+// (the gradient component g, its Nyquist mode dropped, and the axis' part
+// lap of the Laplacian).  A derivative along one axis needs no transform
+// along the others: its multiplier depends on that axis' wave number alone,
+// and |k|^2 is the sum of the three squares (src/toolbox.c:132-139).  The
+// operators are real, so a line of neighbouring pairs (z, z + 1) is
+// transformed as one complex line u + i v and gives (Du, Dv) with no
+// Hermitian split: phi is read and g and lap are written in whole 16-byte
+// pairs, aligned rows.  Geometry: `ls` in units of pairs.  The value phi[0]
+// of the grid's first point is subtracted before the transform (its
+// derivatives vanish): phi is a mean of order 1 with fluctuations of 1e-6 to
+// 1e-2, and every line's transform would round at the size of the mean.  The
+// difference of nearby numbers is exact.  (After the filter the derivatives
+// are those of the filtered field before the mean is added and rounded in,
+// FilterFac.)
+// The bound is HBM traffic, 3 fields of 8 N bytes an axis: both axes at 256^3
+// take 171 us (4.7 TB/s).  The z r2c, y and x fan-out passes of the derivatives
+// through the 3D spectrum, which this replaces, took 307 us.  256-point lines:
+// 16 values a thread in two stages with 296 registers (one wave a SIMD) 171
+// us, 8 values in three stages 183, 16 values held to 256 registers 204, 512
+// lanes a work-group 215.
+// ---------------------------------------------------------------------------
+struct DerivAxis {
+    LineSet ls;
+    const double2 *phi;
+    double2 *g, *lap;
+    double k1, k2;    // 2 pi / (L length), (2 pi / length)^2 / L
+    long rp, rl, rg;  // realization strides of phi, lap, g (pairs)
+};
+
+template <int L, class P, int WG>
+__device__ __forceinline__ void deriv_body(const Blk &bk, double2 *lds,
+                                           const DerivAxis &a,
+                                           const double2 *__restrict__ tw)
+{
+    constexpr int E = P::E, B = StridedShape<L, P, WG>::B, PITCH = Lds<L>::PITCH;
+    const int tid = threadIdx.x;
+    const int b = tid % B, j = tid / B;
+    const long line = (long)bk.x * B + b;
+    const bool act = line < a.ls.nlines;
+    const long base = a.ls.base(act ? line : 0);
+    const double2 *src = a.phi + bk.z * a.rp + base;
+    double2 *gd = a.g + bk.z * a.rg + base, *ld = a.lap + bk.z * a.rl + base;
+    const long st = a.ls.stride;
+    double2 *my = lds + b * PITCH;
+    double2 spec[E];
+    const double phi0 = a.phi[bk.z * a.rp].x;
+    // idle lanes transform line 0 (in bounds) and store nothing
+    auto rd = [&](int, int n) {
+        const double2 v = src[n * st];
+        return make_double2(v.x - phi0, v.y - phi0);
+    };
+    auto keep = [&](int slot, int, double2 v) { spec[slot] = v; };
+    fft_line<L, -1, true, true, P>(my, j, tw, rd, keep);
+    lds_barrier(); // LDS reads of the forward transform are done
+    auto rl = [&](int slot, int n) {
+        const double2 v = spec[chain_slot<L, P>(slot)];
+        const double m = n > L / 2 ? L - n : n, k = -(a.k2 * m * m);
+        return make_double2(v.x * k, v.y * k);
+    };
+    auto wl = [&](int, int n, double2 v) {
+        if (act) ld[n * st] = v;
+    };
+    fft_line<L, +1, true, true, P>(my, j, tw, rl, wl);
+    lds_barrier();
+    auto rg = [&](int slot, int n) {
+        const double2 v = spec[chain_slot<L, P>(slot)];
+        const double k = n > L / 2 ? a.k1 * (n - L) : (2 * n == L ? 0.0 : a.k1 * n);
+        return make_double2(-v.y * k, v.x * k);
+    };
+    auto wg = [&](int, int n, double2 v) {
+        if (act) gd[n * st] = v;
+    };
+    fft_line<L, +1, true, true, P>(my, j, tw, rg, wg);
+}
+
+// Line plans and work-group sizes of the derivative passes
+template <int L> struct DerivPlan { using P = Plan<L>; static constexpr int WG = FFT_WG; };
+
+// both axes (of one length) in one launch: blockIdx.y picks the axis
+struct DerivXY {
+    DerivAxis a[2];
+};
+
+template <int L, class P, int WG>
+__global__ __launch_bounds__(WG) void k_deriv(DerivXY d,
+                                              const double2 *__restrict__ tw)
+{
+    __shared__ double2 lds[StridedShape<L, P, WG>::LDS];
+    deriv_body<L, P, WG>(hw_blk(), lds, d.a[blockIdx.y], tw);
+}
 
 // ---------------------------------------------------------------------------
 // z passes
@@ -362,12 +432,20 @@ __global__ __launch_bounds__(FFT_WG) void k_z_r2c(
     z_r2c_body<L>(hw_blk(), lds, in, out, nrows, rbatch, cbatch, tw, rin, rout);
 }
 
+// A constant kept out of the transform of array 0 of a batch: the c2r pass
+// writes u + *dc to the output and u itself to fl (strides per realization).
+struct ZShift {
+    const double *dc = nullptr;
+    double *fl = nullptr;
+    long rdc = 0, rfl = 0;
+};
+
 // Half rows -> real rows (the c2r z pass).
 template <int L>
 __device__ __forceinline__ void z_c2r_body(
     const Blk &bk, double2 *lds, const double2 *in, double *out, long nrows,
     long cbatch, long rbatch, const double2 *__restrict__ tw, long rin,
-    long rout)
+    long rout, const ZShift &sh)
 {
     using TL = Tile<L>;
     constexpr int MZ = L / 2 + 1;
@@ -388,11 +466,18 @@ __device__ __forceinline__ void z_c2r_body(
     const int w = tid / 64, lane = tid % 64;
     const long row0 = 2 * ((long)bk.x * TL::B + w * TL::LPW);
     const double2 *wl = lds + w * TL::LPW * TL::PITCH;
+    double c = 0.0, *fl = nullptr;
+    if (sh.dc && bk.y == 0) {
+        c = sh.dc[bk.z * sh.rdc];
+        fl = sh.fl + bk.z * sh.rfl;
+    }
     for (int idx = lane; idx < 2 * TL::LPW * L; idx += 64) {
         const int r = idx / L, n = idx - r * L;
         if (row0 + r < nrows) {
             const double2 z = wl[(r >> 1) * TL::PITCH + Lds<L>::idx(n)];
-            stn(out + row0 * L + idx, (r & 1) ? z.y : z.x);
+            const double v = (r & 1) ? z.y : z.x;
+            if (fl) fl[row0 * L + idx] = v;
+            stn(out + row0 * L + idx, v + c);
         }
     }
 }
@@ -400,10 +485,11 @@ __device__ __forceinline__ void z_c2r_body(
 template <int L>
 __global__ __launch_bounds__(FFT_WG) void k_z_c2r(
     const double2 *in, double *out, long nrows, long cbatch, long rbatch,
-    const double2 *__restrict__ tw, long rin, long rout)
+    const double2 *__restrict__ tw, long rin, long rout, ZShift sh)
 {
     __shared__ double2 lds[Tile<L>::B * Tile<L>::PITCH];
-    z_c2r_body<L>(hw_blk(), lds, in, out, nrows, cbatch, rbatch, tw, rin, rout);
+    z_c2r_body<L>(hw_blk(), lds, in, out, nrows, cbatch, rbatch, tw, rin, rout,
+                  sh);
 }
 
 } // namespace ihg

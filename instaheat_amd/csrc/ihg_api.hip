@@ -98,8 +98,8 @@ static void host_filter_axes(const ihg_ctx *c, double *out)
 }
 
 static const char *const FAM_NAMES[F_NFAM] = {
-    "z_r2c", "z_c2r", "y_pass", "x_pass", "x_fanout", "z_c2r_rho", "means",
-    "update_phi_psi", "z_r2c_sources", "y_tt_update_h", "x_roundtrip",
+    "z_r2c", "z_c2r", "y_pass", "x_pass", "xy_deriv", "z_rhs", "means",
+    "update_phi_psi", "y_tt_update_h", "x_roundtrip",
     "observables", "dp_stage", "dp_finish", "rk4", "stream_copy", "dp_dense",
     "gsl_stage", "gsl_finish", "dp_dense_stage"};
 
@@ -309,7 +309,10 @@ static int create_ctx(const ihg_params *p, int nreal, ihg_ctx **out)
         if (rc) return fail(rc);
     }
     // per-realization work arrays of an ensemble, one after the other
-    c->npartials = 3L * 512 * (p->bins > 8 ? p->bins : 8) + 2L * 65536 + 4096;
+    // (the z pass writes one pair of sums per wavefront, at least one pair of
+    // rows each, in work-groups of up to 4 wavefronts)
+    c->npartials = 3L * 512 * (p->bins > 8 ? p->bins : 8) +
+                   std::max(2L * 65536, (long)c->Nx * c->Ny) + 4096;
     if (nreal > 1) {
         c->ens.f = c->Ntot + 1; // even: every realization 16-byte aligned
         c->ens.w = 6 * c->M;
@@ -501,9 +504,9 @@ extern "C" int ihg_mk_rhs(ihg_ctx *c, double t, double *f, double *result,
     c->calls_rhs += 1;
     const int output = (flags & IHG_OUTPUT) ? 1 : 0;
     // with the filter, the filtered spectra of phi and psi are kept for the
-    // derivatives and the output (tmp.phic / tmp.psic, src/toolbox.c:164-171)
+    // output (tmp.phic / tmp.psic, src/toolbox.c:164-171)
     const int kept = (flags & IHG_FILTER) && c->p.enable_filter;
-    if (kept) IHG_TRY(rhs_filter(c, f));
+    if (kept) IHG_TRY(rhs_filter(c, f, output));
     IHG_TRY(rhs_core(c, f, result, output, kept));
     if (c->p.enable_gw) IHG_TRY(rhs_gw(c, f, result));
     if (output) IHG_TRY(rhs_output(c, f, kept));
@@ -572,7 +575,7 @@ extern "C" int ihg_mk_rhs_ensemble(ihg_ctx *c, double t, double *f,
     const int nr = c->nreal;
     c->calls_rhs += nr;
     const int kept = (flags & IHG_FILTER) && c->p.enable_filter;
-    if (kept) IHG_TRY(rhs_filter(c, f, nr));
+    if (kept) IHG_TRY(rhs_filter(c, f, 0, nr));
     IHG_TRY(rhs_core(c, f, result, 0, kept, nr));
     if (c->p.enable_gw) IHG_TRY(rhs_gw(c, f, result, nr));
     return 0;
@@ -624,7 +627,7 @@ extern "C" int ihg_mk_rhs_rk4(ihg_ctx *c, double t, double *f, double *result,
         return ihg_rk4_final(c, d.out, d.k1, d.k2, d.k3, result, d.dt);
     }
     c->calls_rhs += nr;
-    if (kept) IHG_TRY(rhs_filter(c, f, nr));
+    if (kept) IHG_TRY(rhs_filter(c, f, 0, nr));
     IHG_TRY(rhs_core(c, f, result, 0, kept, nr, &d));
     if (c->p.enable_gw) IHG_TRY(rhs_gw(c, f, result, nr, &d));
     return 0;

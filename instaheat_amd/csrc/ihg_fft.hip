@@ -105,17 +105,19 @@ int z_r2c_pass(ihg_ctx *c, const double *in, double2 *out, int batch,
 }
 
 int z_c2r_pass(ihg_ctx *c, const double2 *in, double *out, int batch,
-               long cbatch, long rbatch, int nr, long rin, long rout)
+               long cbatch, long rbatch, int nr, long rin, long rout,
+               const ZShift *sh)
 {
     const long nrows = (long)c->Nx * c->Ny;
     return dispatch_len(c->Nz, [&](auto Lc) {
         constexpr int L = decltype(Lc)::value;
         using TL = Tile<L>;
         dim3 grid((unsigned)((nrows / 2 + TL::B - 1) / TL::B), batch, nr);
-        const double bytes = (8.0 * c->N + 16.0 * c->M) * batch * nr;
+        const double bytes = ((8.0 * c->N + 16.0 * c->M) * batch + (sh ? 8.0 * c->N : 0.0)) * nr;
         return timed(c, F_Z_C2R, bytes, [&]() {
             hipLaunchKernelGGL((k_z_c2r<L>), grid, dim3(FFT_WG), 0, c->stream,
-                               in, out, nrows, cbatch, rbatch, c->tw, rin, rout);
+                               in, out, nrows, cbatch, rbatch, c->tw, rin, rout,
+                               sh ? *sh : ZShift{});
             return hip_check(hipGetLastError(), "k_z_c2r");
         });
     });

@@ -80,7 +80,7 @@ constexpr int fam_lds_max()
                      Fam::template lds<64>(), Fam::template lds<128>()});
 }
 
-// LDS of the strided and fan-out bodies: none for one-stage plans, whose
+// LDS of the strided and derivative bodies: none for one-stage plans, whose
 // only stage loads from and stores to registers
 template <int L>
 constexpr int strided_lds()
@@ -170,13 +170,14 @@ struct FamZC2R {
         long nrows, cbatch, rbatch;
         const double2 *tw;
         long rin, rout;
+        ZShift sh;
     };
     template <int L> static constexpr int lds() { return Tile<L>::B * Tile<L>::PITCH; }
     template <int L>
     __device__ static void run(const Blk &bk, double2 *lds, const Args &a)
     {
         z_c2r_body<L>(bk, lds, a.in, a.out, a.nrows, a.cbatch, a.rbatch, a.tw,
-                      a.rin, a.rout);
+                      a.rin, a.rout, a.sh);
     }
 };
 
@@ -203,55 +204,64 @@ struct FamStrided {
     }
 };
 
-template <int NQ, bool FWD, class Fac>
-struct FamFanout {
-    static constexpr int WG = FFT_WG;
+// the filter round trip along x; WG lanes (RoundtripWG<L>)
+template <int WG_>
+struct FamRoundtrip {
+    static constexpr int WG = WG_;
     static constexpr bool BY_LEN = true;
     struct Args {
-        const double2 *in;
-        double2 *out;
-        long qstride;
+        double2 *data;
         LineSet ls;
         long batch;
         const double2 *tw;
-        Fac fac;
+        FilterFac fac;
         long rr;
+    };
+    template <int L>
+    static constexpr int lds()
+    {
+        return Plan<L>::R1 > 1 ? StridedShape<L, Plan<L>, WG>::LDS : 0;
+    }
+    template <int L>
+    __device__ static void run(const Blk &bk, double2 *lds, const Args &a)
+    {
+        x_roundtrip_body<L, FilterFac, Plan<L>, WG>(bk, lds, a.data, a.ls, a.batch,
+                                                    a.tw, a.fac, a.rr);
+    }
+};
+
+// derivatives along one axis
+struct FamDeriv {
+    static constexpr int WG = FFT_WG;
+    static constexpr bool BY_LEN = true;
+    struct Args {
+        DerivAxis a;
+        const double2 *tw;
     };
     template <int L> static constexpr int lds() { return strided_lds<L>(); }
     template <int L>
     __device__ static void run(const Blk &bk, double2 *lds, const Args &a)
     {
-        x_fanout_body<L, NQ, FWD, Fac, typename FanPlan<L>::P, FanPlan<L>::WG>(
-            bk, lds, a.in, a.out, a.qstride, a.ls, a.batch, a.tw, a.fac, a.rr);
+        deriv_body<L, typename DerivPlan<L>::P, WG>(bk, lds, a.a, a.tw);
     }
 };
 
-struct FamZC2RRho {
+template <bool GW>
+struct FamZRhs {
     static constexpr int WG = FFT_WG;
     static constexpr bool BY_LEN = true;
-    struct Args {
-        const double2 *W;
-        long M;
-        const double *f;
-        double *result, *grad3, *partials;
-        long nrows, N;
-        double m2;
-        const double2 *tw;
-        Ens e;
-    };
-    template <int L> static constexpr int lds() { return z_rho_lds<L>(); }
+    using Args = ZRhsArgs<double2>;
+    template <int L> static constexpr int lds() { return z_rhs_lds<L, WG>(); }
     template <int L>
     __device__ static void run(const Blk &bk, double2 *lds, const Args &a)
     {
-        z_c2r_rho_body<L, double>(bk, lds, a.W, a.M, a.f, a.result, a.grad3,
-                                  nullptr, nullptr, a.partials, a.nrows, a.N,
-                                  a.m2, a.tw, a.e);
+        z_rhs_body<L, GW, double2, WG>(bk, lds, a);
     }
 };
 
 template <bool EP>
 struct FamMeans {
-    static constexpr int WG = RED_WG;
+    static constexpr int WG = MEANS_WG;
     static constexpr bool BY_LEN = false;
     struct Args {
         const double *partials;
@@ -264,7 +274,7 @@ struct FamMeans {
         Ens e;
         Rk4Ep ep;
     };
-    template <int L> static constexpr int lds() { return 4; } // 8 doubles
+    template <int L> static constexpr int lds() { return MEANS_WG / 128; }
     template <int L>
     __device__ static void run(const Blk &bk, double2 *lds, const Args &a)
     {
@@ -282,8 +292,7 @@ struct FamUpdate {
     struct Args {
         const double *f;
         double *result;
-        long N, Ntot;
-        double m2;
+        long N;
         const double *dscal;
         Ens e;
         int nt;
@@ -295,30 +304,10 @@ struct FamUpdate {
     {
         if (a.nt)
             update_phi_psi_body<true, EP>(bk.x, bk.gx, bk.z, a.f, a.result, a.N,
-                                          a.Ntot, a.m2, a.dscal, a.e, a.ep);
+                                          a.dscal, a.e, a.ep);
         else
             update_phi_psi_body<false, EP>(bk.x, bk.gx, bk.z, a.f, a.result,
-                                           a.N, a.Ntot, a.m2, a.dscal, a.e,
-                                           a.ep);
-    }
-};
-
-struct FamSources {
-    static constexpr int WG = FFT_WG;
-    static constexpr bool BY_LEN = true;
-    struct Args {
-        const double *g3;
-        double2 *W;
-        long M, nrows, N;
-        const double2 *tw;
-        long rg, rw;
-    };
-    template <int L> static constexpr int lds() { return Tile<L>::B * Tile<L>::PITCH; }
-    template <int L>
-    __device__ static void run(const Blk &bk, double2 *lds, const Args &a)
-    {
-        z_r2c_sources_body<L, double2>(bk, lds, a.g3, a.W, a.M, a.nrows, a.N,
-                                       a.tw, a.rg, a.rw);
+                                           a.N, a.dscal, a.e, a.ep);
     }
 };
 
@@ -342,6 +331,7 @@ struct FamTT {
         const double2 *tw;
         Ens e;
         long rw;
+        GwAxis ga;
         Rk4Ep ep;
     };
     template <int L>
@@ -354,7 +344,7 @@ struct FamTT {
     {
         y_tt_update_h_body<L, WG, typename GroupTTPlan<L>::P, double2, EP>(
             bk, lds, a.W, a.M, a.f, a.result, a.N, a.Next, a.Ntot, a.kg,
-            a.dscal, a.ls, a.tw, a.e, a.rw, a.ep);
+            a.dscal, a.ls, a.tw, a.e, a.rw, a.ga, a.ep);
     }
 };
 
@@ -504,7 +494,7 @@ static Seg<FamStrided<DIR>> strided_seg(const ihg_ctx *c, double2 *data,
     return s;
 }
 
-// lines per work-group of a z pass and of a strided (fan-out) pass
+// lines per work-group of a z pass and of a strided pass
 static int tile_b(int L)
 {
     return dispatch_len(L, [&](auto Lc) { return Tile<decltype(Lc)::value>::B; });
@@ -607,11 +597,12 @@ static int group_rhs(ihg_group *g, double *const *f, double *const *result,
 
     // mk_ffts_and_filter's filter branch (src/toolbox.c:164-171), as
     // rhs_filter: z r2c, y, x round trip with the window, y, z c2r of the
-    // four fields
+    // four fields (the round trip once per work-group size)
     {
         std::vector<Seg<FamZR2C>> zf;
         std::vector<Seg<FamStrided<-1>>> yf;
-        std::vector<Seg<FamFanout<1, true, FilterFac>>> xf;
+        std::vector<Seg<FamRoundtrip<128>>> xs;
+        std::vector<Seg<FamRoundtrip<256>>> xf;
         std::vector<Seg<FamStrided<+1>>> yb;
         std::vector<Seg<FamZC2R>> zb;
         for (int i = 0; i < n; ++i) {
@@ -624,118 +615,101 @@ static int group_rhs(ihg_group *g, double *const *f, double *const *result,
             zf.push_back({L, gz, {f[i], c->W, nrows, N, M, c->tw, e.f, e.w}});
             yf.push_back(strided_seg<-1>(c, c->W, y_lines_of(c), 4, M));
             const LineSet ls = x_lines_of(c);
-            const FilterFac fac{c->filter, (long)c->Ny * c->Mz, c->Nx, c->Ny,
-                                c->Mz, (double)N, c->W + 4 * M,
-                                nr > 1 ? nullptr : c->Wc,
-                                nr > 1 ? nullptr : c->Wc + M, e.w};
-            const int Bx = strided_b(L);
-            Seg<FamFanout<1, true, FilterFac>> sx;
-            sx.L = L;
-            sx.grid = dim3((unsigned)((ls.nlines + Bx - 1) / Bx), 4, nr);
-            sx.a = {c->W, c->W, 0L, ls, M, c->tw, fac, e.w};
-            xf.push_back(sx);
+            const FilterFac fac = filter_fac(c, 0, nr);
+            const int wg = dispatch_len(L, [&](auto Lc) {
+                return RoundtripWG<decltype(Lc)::value>::WG;
+            });
+            const int Bx = strided_b(L) * wg / FFT_WG;
+            const dim3 gx((unsigned)((ls.nlines + Bx - 1) / Bx), 4, nr);
+            if (wg == 128)
+                xs.push_back({L, gx, {c->W, ls, M, c->tw, fac, e.w}});
+            else
+                xf.push_back({L, gx, {c->W, ls, M, c->tw, fac, e.w}});
             yb.push_back(strided_seg<+1>(c, c->W, y_lines_of(c), 4, M));
-            zb.push_back({L, gz, {c->W, f[i], nrows, M, N, c->tw, e.w, e.f}});
+            zb.push_back({L, gz, {c->W, f[i], nrows, M, N, c->tw, e.w, e.f, filter_shift(c, nr)}});
         }
         IHG_TRY(glaunch(g, zf, "grouped z r2c (filter)"));
         IHG_TRY(glaunch(g, yf, "grouped y pass (filter)"));
         IHG_TRY(glaunch(g, xf, "grouped x round trip (filter)"));
+        IHG_TRY(glaunch(g, xs, "grouped x round trip (filter, 128 lanes)"));
         IHG_TRY(glaunch(g, yb, "grouped y pass (filter)"));
         IHG_TRY(glaunch(g, zb, "grouped z c2r (filter)"));
     }
 
-    // rhs_core: phi_hat (unless the filter kept it), the x fan-out of the
-    // four derivative spectra, y backward, z c2r fused with rho and p, the
-    // means and update_phi_psi (src/toolbox.c:75-299)
+    // rhs_core: the x and y derivatives and the z pass (with the GW sources
+    // or without: the two kinds of contexts have launches of their own, since
+    // a launch's registers are those of its largest body), the means and
+    // update_phi_psi (src/toolbox.c:75-299)
+    std::vector<int> nparts(n);
+    auto scalar_passes = [&](auto gwc) {
+        constexpr bool GW = decltype(gwc)::value;
+        std::vector<Seg<FamDeriv>> dx, dy;
+        std::vector<Seg<FamZRhs<GW>>> zr;
+        for (int i = 0; i < n; ++i) {
+            ihg_ctx *c = g->c[i];
+            if ((c->p.enable_gw != 0) != GW) continue;
+            const int L = c->Nx, nr = c->nreal;
+            const DerivIO io = deriv_io(c, f[i], kept[i], nr);
+            const DerivXY d = deriv_axes(c, io, result[i], nr);
+            const int B = dispatch_len(L, [&](auto Lc) {
+                constexpr int LL = decltype(Lc)::value;
+                return FFT_WG / (LL / DerivPlan<LL>::P::E);
+            });
+            const dim3 gd((unsigned)((d.a[0].ls.nlines + B - 1) / B), 1, nr);
+            dx.push_back({L, gd, {d.a[0], c->tw}});
+            dy.push_back({L, gd, {d.a[1], c->tw}});
+            const ZRhsArgs<double2> za = z_rhs_args<double2>(c, f[i], result[i], io, nr);
+            const unsigned nb = dispatch_len(L, [&](auto Lc) {
+                return (int)z_rhs_blocks<decltype(Lc)::value>(za.nrows, FFT_WG);
+            });
+            nparts[i] = (int)nb * (FFT_WG / 64);
+            if (2L * nparts[i] > c->npartials)
+                return set_error("partials buffer too small");
+            zr.push_back({L, dim3(nb, 1, nr), za});
+        }
+        IHG_TRY(glaunch(g, dx, "grouped x derivatives"));
+        IHG_TRY(glaunch(g, dy, "grouped y derivatives"));
+        return glaunch(g, zr, "grouped z pass");
+    };
+    IHG_TRY(scalar_passes(std::true_type{}));
+    IHG_TRY(scalar_passes(std::false_type{}));
     {
-        std::vector<Seg<FamZR2C>> z1;
-        std::vector<Seg<FamStrided<-1>>> y1;
-        std::vector<Seg<FamFanout<4, true, DerivFac>>> fw;
-        std::vector<Seg<FamFanout<4, false, DerivFac>>> fk;
-        std::vector<Seg<FamStrided<+1>>> yb;
-        std::vector<Seg<FamZC2RRho>> zr;
         std::vector<Seg<FamMeans<EP>>> mn;
         std::vector<Seg<FamUpdate<EP>>> up;
         for (int i = 0; i < n; ++i) {
             ihg_ctx *c = g->c[i];
             const Ens e = ens_of(c);
-            const long N = c->N, M = c->M, nrows = (long)c->Nx * c->Ny;
-            const int L = c->Nx, B = tile_b(L), nr = c->nreal;
-            double2 *W = c->W;
-            if (!kept[i]) {
-                const dim3 gz((unsigned)((nrows / 2 + B - 1) / B), 1, nr);
-                z1.push_back({L, gz, {f[i], W + 4 * M, nrows, 0L, 0L, c->tw, e.f, e.w}});
-                y1.push_back(strided_seg<-1>(c, W + 4 * M, y_lines_of(c), 1, 0L));
-            }
-            const LineSet ls = x_lines_of(c);
-            const DerivFac fac{c->kg, (double)N};
-            const int Bx = strided_b(L);
-            const dim3 gx((unsigned)((ls.nlines + Bx - 1) / Bx), 1, nr);
-            if (kept[i]) {
-                Seg<FamFanout<4, false, DerivFac>> s;
-                s.L = L;
-                s.grid = gx;
-                s.a = {W + 4 * M, W, M, ls, 0L, c->tw, fac, e.w};
-                fk.push_back(s);
-            } else {
-                Seg<FamFanout<4, true, DerivFac>> s;
-                s.L = L;
-                s.grid = gx;
-                s.a = {W + 4 * M, W, M, ls, 0L, c->tw, fac, e.w};
-                fw.push_back(s);
-            }
-            yb.push_back(strided_seg<+1>(c, W, y_lines_of(c), 4, M));
-            const unsigned nb = (unsigned)((2 * nrows + B - 1) / B);
-            if (2L * nb > c->npartials)
-                return set_error("partials buffer too small");
-            const double m2 = c->p.mass * c->p.mass;
-            Seg<FamZC2RRho> sr;
-            sr.L = L;
-            sr.grid = dim3(nb, 1, nr);
-            sr.a = {W, M, f[i], result[i], c->p.enable_gw ? c->grad3 : nullptr,
-                    c->partials, nrows, N, m2, c->tw, e};
-            zr.push_back(sr);
+            const long N = c->N;
+            const int L = c->Nx, nr = c->nreal;
             const Rk4Ep ep = EP ? eps[i] : Rk4Ep{};
             Seg<FamMeans<EP>> sm;
             sm.L = L;
             sm.grid = dim3(nr, 1, 1);
-            sm.a = {c->partials, (int)nb, N, f[i], result[i], c->Ntot, c->dscal,
-                    e, ep};
+            sm.a = {c->partials, nparts[i], N, f[i], result[i], c->Ntot,
+                    c->dscal, e, ep};
             mn.push_back(sm);
             Seg<FamUpdate<EP>> su;
             su.L = L;
             su.grid = dim3(upd_blocks(N), 1, nr);
-            su.a = {f[i], result[i], N, c->Ntot, m2, c->dscal, e,
+            su.a = {f[i], result[i], N, c->dscal, e,
                     4.0 * 8.0 * (double)N * nr >= NT_BYTES ? 1 : 0, ep};
             up.push_back(su);
         }
-        IHG_TRY(glaunch(g, z1, "grouped z r2c"));
-        IHG_TRY(glaunch(g, y1, "grouped y pass"));
-        IHG_TRY(glaunch(g, fw, "grouped x fan-out"));
-        IHG_TRY(glaunch(g, fk, "grouped x fan-out (kept spectrum)"));
-        IHG_TRY(glaunch(g, yb, "grouped y pass"));
-        IHG_TRY(glaunch(g, zr, "grouped z c2r + rho, p"));
         IHG_TRY(glaunch(g, mn, "grouped means"));
         IHG_TRY(glaunch(g, up, "grouped update_phi_psi"));
     }
 
-    // rhs_gw: z r2c of the source products, x pass, the fused y pass +
-    // TT projection + update_h (src/toolbox.c:311-424)
+    // rhs_gw: x pass of the source components, the fused y pass + TT
+    // projection + update_h (src/toolbox.c:311-424)
     {
-        std::vector<Seg<FamSources>> sz;
         std::vector<Seg<FamStrided<-1>>> sx;
         std::vector<Seg<FamTT<EP>>> tt;
         for (int i = 0; i < n; ++i) {
             ihg_ctx *c = g->c[i];
             if (!c->p.enable_gw) continue;
             const Ens e = ens_of(c);
-            const long N = c->N, M = c->M, nrows = (long)c->Nx * c->Ny;
-            const int L = c->Nx, B = tile_b(L), nr = c->nreal;
-            Seg<FamSources> s;
-            s.L = L;
-            s.grid = dim3((unsigned)((nrows + B - 1) / B), 1, nr);
-            s.a = {c->grad3, c->W, M, nrows, N, c->tw, e.g, e.w};
-            sz.push_back(s);
+            const long N = c->N, M = c->M;
+            const int L = c->Nx, nr = c->nreal;
             sx.push_back(strided_seg<-1>(c, c->W, x_lines_of(c), GW_NC, M));
             const LineSet ls = y_lines_of(c);
             const int Bt = dispatch_len(L, [&](auto Lc) {
@@ -746,10 +720,10 @@ static int group_rhs(ihg_group *g, double *const *f, double *const *result,
             st.L = L;
             st.grid = dim3((unsigned)((ls.nlines + Bt - 1) / Bt), 1, nr);
             st.a = {c->W, M, f[i], result[i], N, c->Next, c->Ntot, c->kg,
-                    c->dscal, ls, c->tw, e, e.w, EP ? eps[i] : Rk4Ep{}};
+                    c->dscal, ls, c->tw, e, e.w, gw_axis(c->kg),
+                    EP ? eps[i] : Rk4Ep{}};
             tt.push_back(st);
         }
-        IHG_TRY(glaunch(g, sz, "grouped GW sources"));
         IHG_TRY(glaunch(g, sx, "grouped x pass (sources)"));
         IHG_TRY(glaunch(g, tt, "grouped y pass + TT + update_h"));
     }

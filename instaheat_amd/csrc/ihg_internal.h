@@ -63,8 +63,8 @@ struct KGeom {
 namespace ihg {
 // kernel families timed by the live profiler (ihg_prof_*)
 enum Fam {
-    F_Z_R2C, F_Z_C2R, F_Y_PASS, F_X_PASS, F_X_FANOUT, F_Z_C2R_RHO, F_MEANS,
-    F_UPDATE, F_Z_R2C_SRC, F_TT_UPDATE_H, F_X_ROUNDTRIP, F_OBS, F_DP_STAGE,
+    F_Z_R2C, F_Z_C2R, F_Y_PASS, F_X_PASS, F_DERIV, F_Z_RHS, F_MEANS,
+    F_UPDATE, F_TT_UPDATE_H, F_X_ROUNDTRIP, F_OBS, F_DP_STAGE,
     F_DP_FINISH, F_RK4, F_STREAM_COPY, F_DP_DENSE, F_GSL_STAGE, F_GSL_FINISH,
     F_DP_DENSE_STAGE, F_NFAM
 };
@@ -100,7 +100,7 @@ struct ihg_ctx {
                        // (the mask `filter` of the reference is their min)
     double2 *W;        // 6 spectral work arrays (M complex each)
     double2 *Wc;       // 2 more spectral arrays (phic / psic for output)
-    double *grad3;     // d_x phi, d_y phi, d_z phi (N each) for GW sources
+    double *grad3;     // d_x phi, d_y phi, d_z phi (N each) with GW
     double *rho;       // N
     double *pressure;  // N
     double *tmpf;      // N, Laplacian of psi on output steps (tmp.f)
@@ -133,6 +133,8 @@ struct ihg_ctx {
 
 namespace ihg {
 
+struct ZShift;
+
 // FFT launchers (ihg_fft.hip)
 int fft_r2c(ihg_ctx *c, const double *in, double2 *out, int batch,
             long rbatch, long cbatch);
@@ -149,7 +151,7 @@ int z_r2c_pass(ihg_ctx *c, const double *in, double2 *out, int batch,
                long rout = 0);
 int z_c2r_pass(ihg_ctx *c, const double2 *in, double *out, int batch,
                long cbatch, long rbatch, int nr = 1, long rin = 0,
-               long rout = 0);
+               long rout = 0, const ZShift *sh = nullptr);
 
 // right-hand side launchers (ihg_rhs.hip)
 // scalar slots in ctx->dscal (16 doubles)
@@ -159,6 +161,7 @@ enum {
     S_PHI_MEAN = 2,  // mean of f[0..N) (constraints, psi init)
     S_DPHI_MEAN = 3, // mean of f[N..2N)
     S_DDPHI_MEAN = 4,
+    S_FILTER_DC = 5, // mean of the filtered phi
     S_FEATURES = 8, // a, variance of phi, mean of psi^2 (step proposer)
     S_STAT = 12,    // mean and variance of ihg_mean / ihg_variance
     S_NSCAL = 16
@@ -169,7 +172,8 @@ struct Rk4Ep;
 // nr = 1: one realization (f, result, the work arrays of realization 0);
 // nr = c->nreal: every realization of an ensemble context at once.  ep: the
 // RK4 epilogue of the kernels that write the slope (rk4_fusable contexts)
-int rhs_core(ihg_ctx *c, double *f, double *result, int output, int kept,
+// (filtered: right after rhs_filter on f)
+int rhs_core(ihg_ctx *c, double *f, double *result, int output, int filtered,
              int nr = 1, const Rk4Ep *ep = nullptr);
 // whether the RK4 epilogue is compiled for the context's kernels (FP64, and
 // with GW on y lines of 16 to 128 points)
@@ -178,7 +182,7 @@ int features(ihg_ctx *c, const double *f, double out[3]);
 int default_candidate_x(int len);
 void candidate_counts(const ihg_ctx *c, int n[2]);
 int autotune(ihg_ctx *c, int reps, int out[2], float ms_out[16]);
-int rhs_filter(ihg_ctx *c, double *f, int nr = 1);
+int rhs_filter(ihg_ctx *c, double *f, int output, int nr = 1);
 int rhs_gw(ihg_ctx *c, const double *f, double *result, int nr = 1,
            const Rk4Ep *ep = nullptr);
 int rhs_output(ihg_ctx *c, const double *f, int kept);

@@ -1,20 +1,18 @@
 // ihg_rhs.hip -- the right-hand side mk_rhs (src/toolbox.c:75-626) as fused
 // HIP kernels.
 //
-// Data flow of one call (no filter, no output, GW off):
-//   z r2c pass      phi                  -> W4            (real -> half rows)
-//   y pass          W4                   -> W4            (forward)
-//   x fan-out       W4 -> W0..W3: forward x, times i k_x/N, i k_y/N, i k_z/N,
-//                   -k^2/N, backward x                    (toolbox.c:132-139)
-//   y pass          W0..W3 backward
-//   z c2r + RHS     W0..W3 -> d_i phi, lap phi in LDS; rho, p, block sums;
-//                   writes lap -> result[N..2N), p -> result[3N..4N)
-//                                                         (toolbox.c:140-243)
+// Data flow of one call (no filter, no output):
+//   derivatives     phi -> d_x phi, d_xx phi and d_y phi, d_yy phi, each from
+//                   transforms along its own axis       (toolbox.c:132-139)
+//   z pass          phi, its x and y derivatives, dphi, psi -> p, the part of
+//                   the slope of dphi without means, block sums of rho and p;
+//                   with GW the z r2c of five source products (pairs of rows
+//                   in one complex row)                 (toolbox.c:140-243)
 //   means           block sums -> rho_mean, pressure_mean, da   (:87, :241)
-//   update          result[0..4N) from f, lap, p, means   (toolbox.c:282-299)
-// GW on adds: z r2c of five products of d_i phi d_j phi (pairs in one complex
-// row), an x pass, and one y pass that also does the TT projection and the h
-// update (toolbox.c:311-424).
+//   update          result[0..4N)                       (toolbox.c:282-299)
+// GW on adds an x pass of the source components and one y pass that also does
+// the TT projection and the h update (toolbox.c:311-424).
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 #include <type_traits>
@@ -36,22 +34,22 @@ static inline unsigned nblocks(long n, int per_block, unsigned cap)
 }
 
 // rho_mean, pressure_mean and da of every realization (one work-group each)
-__global__ __launch_bounds__(RED_WG) void k_means(
+__global__ __launch_bounds__(MEANS_WG) void k_means(
     const double *__restrict__ partials, int nparts, long N,
     const double *__restrict__ f, double *__restrict__ result, long Ntot,
     double *__restrict__ dscal, Ens e)
 {
-    __shared__ double sh[8];
+    __shared__ double sh[MEANS_WG / 64];
     means_body(blockIdx.x, sh, partials, nparts, N, f, result, Ntot, dscal, e);
 }
 
 // the same three kernels with the RK4 epilogue of their slopes
-__global__ __launch_bounds__(RED_WG) void k_means_rk4(
+__global__ __launch_bounds__(MEANS_WG) void k_means_rk4(
     const double *__restrict__ partials, int nparts, long N,
     const double *__restrict__ f, double *__restrict__ result, long Ntot,
     double *__restrict__ dscal, Ens e, Rk4Ep ep)
 {
-    __shared__ double sh[8];
+    __shared__ double sh[MEANS_WG / 64];
     means_body<true>(blockIdx.x, sh, partials, nparts, N, f, result, Ntot,
                      dscal, e, ep);
 }
@@ -59,10 +57,10 @@ __global__ __launch_bounds__(RED_WG) void k_means_rk4(
 template <bool NT>
 __global__ __launch_bounds__(RED_WG) void k_update_phi_psi_rk4(
     const double *__restrict__ f, double *__restrict__ result, long N,
-    long Ntot, double m2, const double *__restrict__ dscal, Ens e, Rk4Ep ep)
+    const double *__restrict__ dscal, Ens e, Rk4Ep ep)
 {
     update_phi_psi_body<NT, true>(blockIdx.x, gridDim.x, blockIdx.z, f, result,
-                                  N, Ntot, m2, dscal, e, ep);
+                                  N, dscal, e, ep);
 }
 
 template <int L, int WG, class P>
@@ -70,12 +68,12 @@ __global__ __launch_bounds__(WG) void k_y_tt_update_h_rk4(
     const double2 *W, long M, const double *__restrict__ f,
     double *__restrict__ result, long N, long Next, long Ntot, KGeom kg,
     const double *__restrict__ dscal, LineSet ls,
-    const double2 *__restrict__ tw, Ens e, long rw, Rk4Ep ep)
+    const double2 *__restrict__ tw, Ens e, long rw, GwAxis ga, Rk4Ep ep)
 {
     __shared__ double2 lds[tt_lds<L, WG, P>()];
     y_tt_update_h_body<L, WG, P, double2, true>(hw_blk(), lds, W, M, f, result,
                                                 N, Next, Ntot, kg, dscal, ls,
-                                                tw, e, rw, ep);
+                                                tw, e, rw, ga, ep);
 }
 
 // the y line lengths whose TT pass has the RK4 epilogue compiled in
@@ -108,82 +106,168 @@ static LineSet x_lineset(const ihg_ctx *c)
     return LineSet{plane, plane, 0, plane};
 }
 
-int rhs_core(ihg_ctx *c, double *f, double *result, int output, int kept,
+// The x and y gradients go to grad3 where the FP64 GW source keeps them; else
+// to W + 3M and W + 4M, which nothing else uses during the z pass (the FP32
+// source components fill less than the first half of W).  The filtered
+// fluctuations of phi are in W + 5M, past the filter's four spectra and the
+// five FP64 source components.
+DerivIO deriv_io(const ihg_ctx *c, const double *f, int filtered, int nr)
+{
+    auto at = [&](int k) { return reinterpret_cast<double *>(c->W + k * c->M); };
+    const bool many = nr > 1;
+    const long rw = many ? 2 * c->ens.w : 0;
+    DerivIO io{f, nullptr, nullptr, nullptr, many ? c->ens.f : 0, 0, rw};
+    if (filtered) {
+        io.phi = at(5);
+        io.rphi = rw;
+        io.dc = c->dscal + S_FILTER_DC;
+        io.rdc = many ? c->ens.s : 0;
+    }
+    if (c->p.enable_gw && !c->p.gw_fp32) {
+        io.gx = c->grad3;
+        io.gy = c->grad3 + c->N;
+        io.rxy = many ? c->ens.g : 0;
+    } else {
+        io.gx = at(3);
+        io.gy = at(4);
+    }
+    return io;
+}
+
+// x and y derivative passes (pairs of z neighbours as complex values); the
+// second derivatives go to result[N..2N) (x) and result[2N..3N) (y)
+DerivXY deriv_axes(const ihg_ctx *c, const DerivIO &io, double *result, int nr)
+{
+    const long nzp = c->Nz / 2, plane = (long)c->Ny * nzp;
+    const long rl = nr > 1 ? c->ens.f / 2 : 0;
+    auto d2 = [](double *p) { return reinterpret_cast<double2 *>(p); };
+    const double2 *phi = reinterpret_cast<const double2 *>(io.phi);
+    DerivXY d;
+    d.a[0] = DerivAxis{LineSet{plane, plane, 0, plane}, phi, d2(io.gx),
+                       d2(result + c->N), c->kg.kx1 / c->Nx, c->kg.kx2 / c->Nx,
+                       io.rphi / 2, rl, io.rxy / 2};
+    d.a[1] = DerivAxis{LineSet{c->Nx * nzp, nzp, plane, nzp}, phi, d2(io.gy),
+                       d2(result + 2 * c->N), c->kg.ky1 / c->Ny,
+                       c->kg.ky2 / c->Ny, io.rphi / 2, rl, io.rxy / 2};
+    return d;
+}
+
+FilterFac filter_fac(const ihg_ctx *c, int output, int nr)
+{
+    return FilterFac{c->filter, (long)c->Ny * c->Mz, c->Nx, c->Ny, c->Mz,
+                     (double)c->N, output ? c->Wc : nullptr,
+                     output ? c->Wc + c->M : nullptr, c->dscal + S_FILTER_DC,
+                     nr > 1 ? c->ens.s : 0};
+}
+
+ZShift filter_shift(const ihg_ctx *c, int nr)
+{
+    ZShift z;
+    z.dc = c->dscal + S_FILTER_DC;
+    z.fl = reinterpret_cast<double *>(c->W + 5 * c->M);
+    z.rdc = nr > 1 ? c->ens.s : 0;
+    z.rfl = nr > 1 ? 2 * c->ens.w : 0;
+    return z;
+}
+
+// Work-group size of the derivative and z passes: single wavefronts while
+// 256 lanes a work-group would leave CUs idle.
+static int small_wg(long blocks256) { return blocks256 < 512 ? 64 : 256; }
+
+template <int L, int WG>
+static int launch_deriv(ihg_ctx *c, const DerivXY &d, int naxes, int nr)
+{
+    using P = typename DerivPlan<L>::P;
+    constexpr int B = WG / (L / P::E);
+    const long nl = naxes == 2 ? std::max(d.a[0].ls.nlines, d.a[1].ls.nlines)
+                               : d.a[0].ls.nlines;
+    const dim3 grid((unsigned)((nl + B - 1) / B), naxes, nr);
+    hipLaunchKernelGGL((k_deriv<L, P, WG>), grid, dim3(WG), 0, c->stream, d,
+                       c->tw);
+    return hip_check(hipGetLastError(), "k_deriv");
+}
+
+static int deriv_pass(ihg_ctx *c, int len, const DerivXY &d, int naxes, int nr)
+{
+    return dispatch_len(len, [&](auto Lc) {
+        constexpr int L = decltype(Lc)::value;
+        using P = typename DerivPlan<L>::P;
+        constexpr int WG = DerivPlan<L>::WG, B = WG / (L / P::E);
+        return timed(c, F_DERIV, 24.0 * c->N * naxes * nr, [&]() {
+            if constexpr (L / P::E <= 64)
+                if (small_wg((d.a[0].ls.nlines + B - 1) / B * naxes * nr) == 64)
+                    return launch_deriv<L, 64>(c, d, naxes, nr);
+            return launch_deriv<L, WG>(c, d, naxes, nr);
+        });
+    });
+}
+
+template <class C>
+static int z_pass(ihg_ctx *c, const double *f, double *result, int output,
+                  const DerivIO &io, int nr, int &nparts)
+{
+    const bool gw = c->p.enable_gw != 0;
+    ZRhsArgs<C> a = z_rhs_args<C>(c, f, result, io, nr);
+    if (output) {
+        a.rho = c->rho;
+        a.pressure = c->pressure;
+    }
+    return dispatch_len(c->Nz, [&](auto Lc) {
+        constexpr int L = decltype(Lc)::value;
+        const unsigned nb = z_rhs_blocks<L>(a.nrows, 256);
+        const int wg = small_wg((long)nb * nr);
+        const dim3 grid(wg == 64 ? z_rhs_blocks<L>(a.nrows, 64) : nb, 1, nr);
+        nparts = (int)grid.x * (wg / 64);
+        if (2L * nparts > c->npartials)
+            return set_error("partials buffer too small");
+        // phi, dphi, psi, two gradients, two second derivatives in; A, p
+        // (rho and p on output calls, gradients and sources with GW) out
+        const double rs = sizeof(typename CT<C>::R);
+        const double bytes =
+            (8.0 * c->N * (9 + (output ? 2 : 0)) +
+             (gw ? (rs == 4 ? 3.0 : 1.0) * rs * c->N + GW_NC * sizeof(C) * c->M : 0.0)) * nr;
+        return timed(c, F_Z_RHS, bytes, [&]() {
+            auto go = [&](auto gwc) {
+                constexpr bool G = decltype(gwc)::value;
+                if (wg == 64)
+                    hipLaunchKernelGGL((k_z_rhs<L, G, C, 64>), grid, dim3(64), 0, c->stream, a);
+                else
+                    hipLaunchKernelGGL((k_z_rhs<L, G, C, 256>), grid, dim3(256), 0, c->stream, a);
+            };
+            if (gw)
+                go(std::true_type{});
+            else if constexpr (sizeof(typename CT<C>::R) == 8)
+                go(std::false_type{});
+            return hip_check(hipGetLastError(), "k_z_rhs");
+        });
+    });
+}
+
+int rhs_core(ihg_ctx *c, double *f, double *result, int output, int filtered,
              int nr, const Rk4Ep *ep)
 {
-    const long N = c->N, M = c->M;
-    const double Nd = (double)N;
-    const double m2 = c->p.mass * c->p.mass;
-    double2 *W = c->W;
+    const long N = c->N;
     const Ens e = nr > 1 ? c->ens : Ens{};
-    // phi_hat into W4: kept by the filter pass (full spectrum), or here by
-    // the z and y passes (the x pass is the fan-out's first half)
-    if (!kept) {
-        IHG_TRY(z_r2c_pass(c, f, W + 4 * M, 1, 0, 0, nr, e.f, e.w));
-        IHG_TRY(y_pass(c, W + 4 * M, -1, 1, 0, nr, e.w));
+    const DerivIO io = deriv_io(c, f, filtered, nr);
+    const DerivXY d = deriv_axes(c, io, result, nr);
+    if (c->Nx == c->Ny) {
+        IHG_TRY(deriv_pass(c, c->Nx, d, 2, nr));
+    } else {
+        IHG_TRY(deriv_pass(c, c->Nx, d, 1, nr));
+        IHG_TRY(deriv_pass(c, c->Ny, DerivXY{{d.a[1], d.a[0]}}, 1, nr));
     }
-    // x fan-out into the four derivative spectra W0..W3
-    IHG_TRY(dispatch_len(c->Nx, [&](auto Lc) {
-        constexpr int L = decltype(Lc)::value;
-        using FP = FanPlan<L>;
-        using P = typename FP::P;
-        constexpr int B = FP::WG / (L / P::E);
-        const LineSet ls = x_lineset(c);
-        DerivFac fac{c->kg, Nd};
-        const dim3 grid((unsigned)((ls.nlines + B - 1) / B), 1, nr);
-        return timed(c, F_X_FANOUT, 5.0 * 16.0 * M * nr, [&]() {
-            if (kept)
-                hipLaunchKernelGGL((k_x_fanout<L, 4, false, DerivFac, P, FP::WG>),
-                                   grid, dim3(FP::WG), 0, c->stream, W + 4 * M,
-                                   W, M, ls, 0L, c->tw, fac, e.w);
-            else
-                hipLaunchKernelGGL((k_x_fanout<L, 4, true, DerivFac, P, FP::WG>),
-                                   grid, dim3(FP::WG), 0, c->stream, W + 4 * M,
-                                   W, M, ls, 0L, c->tw, fac, e.w);
-            return hip_check(hipGetLastError(), "k_x_fanout");
-        });
-    }));
-    IHG_TRY(y_pass(c, W, +1, 4, M, nr, e.w));
-    const long nrows = (long)c->Nx * c->Ny;
-    const bool gw = c->p.enable_gw != 0;
     int nparts = 0;
-    IHG_TRY(dispatch_len(c->Nz, [&](auto Lc) {
-        constexpr int L = decltype(Lc)::value;
-        using TL = Tile<L>;
-        const unsigned nb = (unsigned)((2 * nrows + TL::B - 1) / TL::B);
-        nparts = (int)nb;
-        if (2L * nb > c->npartials)
-            return set_error("partials buffer too small");
-        // 4 spectra in; phi, dphi, psi in; lap, p out (+ gradients, rho, p)
-        const double gbytes = (gw && c->p.gw_fp32) ? 4.0 : 8.0;
-        const double bytes = (4.0 * 16.0 * M + 8.0 * N * (5 + (output ? 2 : 0)) +
-                              (gw ? 3.0 * gbytes * N : 0.0)) * nr;
-        const dim3 grid(nb, 1, nr);
-        return timed(c, F_Z_C2R_RHO, bytes, [&]() {
-            if (gw && c->p.gw_fp32)
-                hipLaunchKernelGGL((k_z_c2r_rho<L, float>), grid,
-                                   dim3(FFT_WG), 0, c->stream, W, M, f, result,
-                                   reinterpret_cast<float *>(c->grad3),
-                                   output ? c->rho : nullptr,
-                                   output ? c->pressure : nullptr, c->partials,
-                                   nrows, N, m2, c->tw, e);
-            else
-                hipLaunchKernelGGL((k_z_c2r_rho<L, double>), grid,
-                                   dim3(FFT_WG), 0, c->stream, W, M, f, result,
-                                   gw ? c->grad3 : nullptr,
-                                   output ? c->rho : nullptr,
-                                   output ? c->pressure : nullptr, c->partials,
-                                   nrows, N, m2, c->tw, e);
-            return hip_check(hipGetLastError(), "k_z_c2r_rho");
-        });
-    }));
+    if (c->p.enable_gw && c->p.gw_fp32)
+        IHG_TRY(z_pass<float2>(c, f, result, output, io, nr, nparts));
+    else
+        IHG_TRY(z_pass<double2>(c, f, result, output, io, nr, nparts));
     IHG_TRY(timed(c, F_MEANS, 16.0 * nparts * nr, [&]() {
         if (ep)
-            hipLaunchKernelGGL(k_means_rk4, dim3(nr), dim3(RED_WG), 0,
+            hipLaunchKernelGGL(k_means_rk4, dim3(nr), dim3(MEANS_WG), 0,
                                c->stream, c->partials, nparts, N, f, result,
                                c->Ntot, c->dscal, e, *ep);
         else
-            hipLaunchKernelGGL(k_means, dim3(nr), dim3(RED_WG), 0, c->stream,
+            hipLaunchKernelGGL(k_means, dim3(nr), dim3(MEANS_WG), 0, c->stream,
                                c->partials, nparts, N, f, result, c->Ntot,
                                c->dscal, e);
         return hip_check(hipGetLastError(), "k_means");
@@ -191,7 +275,7 @@ int rhs_core(ihg_ctx *c, double *f, double *result, int output, int kept,
     // the epilogue reads y (and k1..k3) and writes the stage output beside
     // the slope: 2 (stage) or 4 (final, no slope written) more blocks
     const double ep_blocks = !ep ? 0.0 : (ep->mode == RK4_FINAL ? 4.0 : 8.0);
-    return timed(c, F_UPDATE, (10.0 + ep_blocks) * 8.0 * N * nr, [&]() {
+    return timed(c, F_UPDATE, (9.0 + ep_blocks) * 8.0 * N * nr, [&]() {
         // the streaming hint when the four blocks of all realizations
         // outgrow the caches
         const bool nt = 4.0 * 8.0 * (double)N * nr >= NT_BYTES;
@@ -200,39 +284,26 @@ int rhs_core(ihg_ctx *c, double *f, double *result, int output, int kept,
             hipLaunchKernelGGL((nt ? k_update_phi_psi_rk4<true>
                                    : k_update_phi_psi_rk4<false>),
                                grid, dim3(RED_WG), 0, c->stream, f, result, N,
-                               c->Ntot, m2, c->dscal, e, *ep);
+                               c->dscal, e, *ep);
         else
             hipLaunchKernelGGL((nt ? k_update_phi_psi<true>
                                    : k_update_phi_psi<false>),
                                grid, dim3(RED_WG), 0, c->stream, f, result, N,
-                               c->Ntot, m2, c->dscal, e);
+                               c->dscal, e);
         return hip_check(hipGetLastError(), "k_update_phi_psi");
     });
 }
 
-// GW source pipeline on complex type C: z r2c of the products, x pass,
-// fused y pass + TT + update_h.  Wk holds 6 M values of C, g3 the gradients;
-// realization r of an ensemble finds them r * rw and r * rg further on.
+// GW source pipeline on complex type C after the z pass: x pass, fused y
+// pass + TT + update_h.  Wk holds 6 M values of C; realization r of an
+// ensemble finds them r * rw further on.
 template <class C>
-static int rhs_gw_t(ihg_ctx *c, const typename CT<C>::R *g3, C *Wk,
-                    const C *tw, const double *f, double *result, int nr,
-                    long rg, long rw, const Rk4Ep *ep)
+static int rhs_gw_t(ihg_ctx *c, C *Wk, const C *tw, const double *f,
+                    double *result, int nr, long rw, const Rk4Ep *ep)
 {
     const long N = c->N, M = c->M;
-    const long nrows = (long)c->Nx * c->Ny;
-    const double cs = sizeof(C), rs = sizeof(typename CT<C>::R);
+    const double cs = sizeof(C);
     const Ens e = nr > 1 ? c->ens : Ens{};
-    IHG_TRY(dispatch_len(c->Nz, [&](auto Lc) {
-        constexpr int L = decltype(Lc)::value;
-        using TL = Tile<L>;
-        const unsigned nb = (unsigned)((nrows + TL::B - 1) / TL::B);
-        return timed(c, F_Z_R2C_SRC, (3.0 * rs * N + GW_NC * cs * M) * nr, [&]() {
-            hipLaunchKernelGGL((k_z_r2c_sources<L, C>), dim3(nb, 1, nr),
-                               dim3(FFT_WG), 0, c->stream, g3, Wk, M, nrows, N,
-                               tw, rg, rw);
-            return hip_check(hipGetLastError(), "k_z_r2c_sources");
-        });
-    }));
     if constexpr (std::is_same<C, float2>::value)
         IHG_TRY(x_pass_f32(c, Wk, -1, GW_NC, M, nr, rw));
     else
@@ -252,7 +323,7 @@ static int rhs_gw_t(ihg_ctx *c, const typename CT<C>::R *g3, C *Wk,
                     hipLaunchKernelGGL((k_y_tt_update_h_rk4<L, TP::WG, typename TP::P>),
                                        dim3(nb, 1, nr), dim3(TP::WG), 0, c->stream, Wk,
                                        M, f, result, N, c->Next, c->Ntot, c->kg,
-                                       c->dscal, ls, tw, e, rw, *ep);
+                                       c->dscal, ls, tw, e, rw, gw_axis(c->kg), *ep);
                     return hip_check(hipGetLastError(), "k_y_tt_update_h_rk4");
                 });
             });
@@ -270,7 +341,7 @@ static int rhs_gw_t(ihg_ctx *c, const typename CT<C>::R *g3, C *Wk,
             hipLaunchKernelGGL((k_y_tt_update_h<L, TP::WG, typename TP::P, C>),
                                dim3(nb, 1, nr), dim3(TP::WG), 0, c->stream, Wk,
                                M, f, result, N, c->Next, c->Ntot, c->kg,
-                               c->dscal, ls, tw, e, rw);
+                               c->dscal, ls, tw, e, rw, gw_axis(c->kg));
             return hip_check(hipGetLastError(), "k_y_tt_update_h");
         });
     });
@@ -279,22 +350,19 @@ static int rhs_gw_t(ihg_ctx *c, const typename CT<C>::R *g3, C *Wk,
 int rhs_gw(ihg_ctx *c, const double *f, double *result, int nr,
            const Rk4Ep *ep)
 {
-    const Ens e = nr > 1 ? c->ens : Ens{};
+    const long rw = nr > 1 ? c->ens.w : 0;
     if (c->p.gw_fp32)
-        // FP32 values in the FP64 buffers: 6 M float2 fit in W, 3 N floats
-        // in grad3 (the same element strides per realization)
-        return rhs_gw_t<float2>(c, reinterpret_cast<const float *>(c->grad3),
-                                reinterpret_cast<float2 *>(c->W), c->twf, f,
-                                result, nr, e.g, e.w, ep);
-    return rhs_gw_t<double2>(c, c->grad3, c->W, c->tw, f, result, nr, e.g,
-                             e.w, ep);
+        // FP32 values in the FP64 buffer, realizations at the same addresses
+        return rhs_gw_t<float2>(c, reinterpret_cast<float2 *>(c->W), c->twf, f,
+                                result, nr, 2 * rw, ep);
+    return rhs_gw_t<double2>(c, c->W, c->tw, f, result, nr, rw, ep);
 }
 
 // mk_ffts_and_filter's filter branch (src/toolbox.c:164-171): phi, dphi,
-// psi, dpsi (contiguous in f) filtered in place, all four in one batch.
-// The filtered spectra of phi (-> W4 for the derivatives and Wc for the
-// output) and psi (-> Wc + M) are kept, as the reference keeps them.
-int rhs_filter(ihg_ctx *c, double *f, int nr)
+// psi, dpsi (contiguous in f) filtered in place, all four in one batch.  An
+// output call keeps the filtered spectra of phi (Wc) and psi (Wc + M); the
+// fluctuations of the filtered phi stay in W + 5M for rhs_core.
+int rhs_filter(ihg_ctx *c, double *f, int output, int nr)
 {
     const long N = c->N, M = c->M;
     double2 *W = c->W;
@@ -303,24 +371,20 @@ int rhs_filter(ihg_ctx *c, double *f, int nr)
     IHG_TRY(y_pass(c, W, -1, 4, M, nr, e.w));
     IHG_TRY(dispatch_len(c->Nx, [&](auto Lc) {
         constexpr int L = decltype(Lc)::value;
-        using SS = StridedShape<L>;
+        constexpr int WG = RoundtripWG<L>::WG;
+        using SS = StridedShape<L, Plan<L>, WG>;
         const LineSet ls = x_lineset(c);
-        // one realization: keep phi_hat in W4 and Wc, psi_hat in Wc + M;
-        // an ensemble (no output calls) keeps phi_hat in each W4
-        FilterFac fac{c->filter, (long)c->Ny * c->Mz, c->Nx, c->Ny, c->Mz,
-                      (double)N, W + 4 * M, nr > 1 ? nullptr : c->Wc,
-                      nr > 1 ? nullptr : c->Wc + M, e.w};
-        // four fields in and out, three kept spectra out
-        return timed(c, F_X_ROUNDTRIP, 11.0 * 16.0 * M * nr, [&]() {
-            hipLaunchKernelGGL((k_x_fanout<L, 1, true, FilterFac>),
+        const FilterFac fac = filter_fac(c, output, nr);
+        return timed(c, F_X_ROUNDTRIP, (output ? 10.0 : 8.0) * 16.0 * M * nr, [&]() {
+            hipLaunchKernelGGL((k_x_roundtrip<L, FilterFac, Plan<L>, WG>),
                                dim3((unsigned)((ls.nlines + SS::B - 1) / SS::B), 4, nr),
-                               dim3(FFT_WG), 0, c->stream, W, W, 0L, ls, M,
-                               c->tw, fac, e.w);
-            return hip_check(hipGetLastError(), "k_x_fanout (filter)");
+                               dim3(WG), 0, c->stream, W, ls, M, c->tw, fac, e.w);
+            return hip_check(hipGetLastError(), "k_x_roundtrip");
         });
     }));
     IHG_TRY(y_pass(c, W, +1, 4, M, nr, e.w));
-    return z_c2r_pass(c, W, f, 4, M, N, nr, e.w, e.f);
+    const ZShift sh = filter_shift(c, nr);
+    return z_c2r_pass(c, W, f, 4, M, N, nr, e.w, e.f, &sh);
 }
 
 } // namespace ihg

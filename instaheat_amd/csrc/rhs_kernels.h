@@ -18,42 +18,24 @@
 
 namespace ihg {
 
-// ---------------------------------------------------------------------------
-// spectral derivative factors (mk_gradient_squared_and_laplacian,
-// src/toolbox.c:132-139): pre = phi_hat / N; outputs pre * i * k_x,
-// pre * i * k_y, pre * i * k_z (Nyquist-zeroed) and -pre * k^2
-// ---------------------------------------------------------------------------
-struct DerivFac {
-    KGeom kg;
-    double Nd;
-    __device__ double2 operator()(Blk, int q, long line, int n,
-                                  double2 v) const
-    {
-        const int iy = (int)(line / kg.Mz), iz = (int)(line - (long)iy * kg.Mz);
-        const double2 pre = make_double2(v.x / Nd, v.y / Nd);
-        if (q == 3) {
-            const double ks = kg.ksq(n, iy, iz);
-            return make_double2(-(pre.x * ks), -(pre.y * ks));
-        }
-        const double k = (q == 0) ? kg.kxd(n) : ((q == 1) ? kg.kyd(iy) : kg.kzd(iz));
-        return make_double2(-pre.y * k, pre.x * k);
-    }
-};
-
 // capply_filter (src/toolbox.c:616-626): in *= filter; out = in / N.
-// The filtered spectra in *= filter of phi (batch 0) and psi (batch 2) are
-// kept, as mk_ffts_and_filter keeps tmp.phic / tmp.psic
-// (src/toolbox.c:164-171): phi's in keep_phi (and keep_phi2), psi's in
-// keep_psi; null pointers keep nothing.
+// An output call keeps the filtered spectra of phi (batch 0) and psi (batch
+// 2), as mk_ffts_and_filter keeps tmp.phic / tmp.psic (src/toolbox.c:164-
+// 171): null pointers keep nothing.
+// The mean of phi (its k = 0 mode) goes to *dc instead of the backward
+// transform, and the c2r pass adds it (ZShift): so the right-hand side has
+// the filtered fluctuations without the rounding of phi, which is of order 1,
+// to double precision -- the reference differentiates the kept spectrum, not
+// the rounded field.
 struct FilterFac {
     const double *__restrict__ filt; // Fx[Nx] | Fy[Ny] | Fz[Mz]
     long plane; // Ny * Mz
     int Nx, Ny, Mz;
     double Nd;
-    double2 *keep_phi, *keep_phi2, *keep_psi;
-    long rkeep; // realization stride of keep_phi (ensembles)
-    __device__ double2 operator()(Blk bk, int, long line, int n,
-                                  double2 v) const
+    double2 *keep_phi, *keep_psi;
+    double *dc; // mean of the filtered phi per realization, rdc apart
+    long rdc;
+    __device__ double2 operator()(Blk bk, long line, int n, double2 v) const
     {
         const bool in = line < plane; // padding lines read entry 0
         const long lc = in ? line : 0;
@@ -62,153 +44,391 @@ struct FilterFac {
         const int j = (int)(lc / Mz), k = (int)(lc - (long)j * Mz);
         const double F = fmin(fmin(filt[n], filt[Nx + j]), filt[Nx + Ny + k]);
         const double2 w = make_double2(v.x * F, v.y * F);
-        if (in && bk.y == 0 && keep_phi) {
-            keep_phi[bk.z * rkeep + i] = w;
-            if (keep_phi2) keep_phi2[i] = w;
-        }
+        if (in && bk.y == 0 && keep_phi)
+            keep_phi[i] = w;
         if (in && bk.y == 2 && keep_psi)
             keep_psi[i] = w;
+        if (bk.y == 0 && line == 0 && n == 0) {
+            dc[bk.z * rdc] = w.x / Nd;
+            return make_double2(0.0, 0.0);
+        }
         return make_double2(w.x / Nd, w.y / Nd);
     }
 };
 
-// LDS of the z c2r + rho pass in complex values: the tile's lines, then the
-// L stage twiddles
-template <int L>
-__host__ __device__ constexpr int z_rho_lines()
+// ---------------------------------------------------------------------------
+// The z pass of the right-hand side.  A complex line is a pair of rows A + i
+// B of phi (the z derivatives are real operators, so no Hermitian split):
+// forward transform, d_z phi and d_zz phi by two backward ones, then with the
+// x and y derivatives (k_deriv) assemble_gradient_squared and mk_rho_and_p
+// (src/toolbox.c:196-243): block sums of rho and p, p and the part of the
+// slope of dphi that needs no mean,
+//   A = (1 + 4 psi) lap phi / a^2 - (1 + 2 psi) m^2 phi   (toolbox.c:282-299)
+// With GW also the z r2c of the source products: the three gradients are in
+// registers at that point, so they are neither written and read again (d_z
+// phi is written, for ihg_aux) nor packed with a wasted half line.
+//
+// GW sources (mk_gw_sources, src/toolbox.c:410-424): only the transverse
+// traceless part of d_i phi d_j phi enters the equations, and the projection
+// takes delta_ij s to 0 for every s (P is a projector of trace 2 built from
+// the full k with k_i k_i = k^2), so one diagonal product, that of axis
+// GwAxis::m, is subtracted from the other two: GW_NC = 5 components instead of
+// six, (xx - mm, xy, xz, yy - mm, yz) with zz - mm in the place of the one
+// that vanishes (two DOPRI853 steps at 256^3 86.0 -> 83.9 ms).  m is the axis
+// of the smallest Nyquist wave number, so that a difference is not rounded at
+// the size of a much larger product: with m = z on a box resolved more finely
+// along z the slopes of h lost a factor of 2.5 (FP32, 4 x 4 x 512 points on a
+// cube).
+// Component c of rows A and B is one complex line; its half rows go to W + c M.
+//
+// A line's T threads are lanes of one wavefront and every wavefront works
+// alone (its own LDS lines and its own pair of partial sums), so there is no
+// work-group barrier, and the work-group size changes no value: 64 lanes
+// spread a small grid over more CUs, 256 share the twiddle table.
+//
+// Measured at 256^3 with GW: 411 us for the 15 fields' worth of traffic (8 N
+// bytes each; 4.9 TB/s), with the FP32 source 401 us for 13, so neither HBM
+// alone nor the arithmetic bounds it; the y c2c, z c2r + rho and z r2c passes
+// that it replaces moved 31 and took 780 us.  4 values a thread (3 waves a
+// SIMD) against 8 (2 waves): 411 against 415 us at 256^3, 278 against 341 us
+// for 4 x 128^3, 5.1 against 9.3 us for one 32^3 grid without GW.
+// ---------------------------------------------------------------------------
+constexpr int GW_NC = 5;
+
+// The axis (0, 1, 2) whose diagonal product is subtracted from the others:
+// the one of the smallest Nyquist wave number, z where they are equal.
+struct GwAxis {
+    int m;
+};
+inline GwAxis gw_axis(const KGeom &kg)
 {
-    return Tile<L>::B * Tile<L>::PITCH;
-}
-template <int L>
-__host__ __device__ constexpr int z_rho_lds()
-{
-    return z_rho_lines<L>() + L;
+    const double kx = kg.kx1 * kg.Nx, ky = kg.ky1 * kg.Ny, kz = kg.kz1 * kg.Nz;
+    GwAxis a{2};
+    double least = kz;
+    if (kx < least) { a.m = 0; least = kx; }
+    if (ky < least) a.m = 1;
+    return a;
 }
 
-// ---------------------------------------------------------------------------
-// z c2r of the four derivative spectra fused with assemble_gradient_squared
-// and mk_rho_and_p (src/toolbox.c:196-243).  Line 2r holds (d_x, d_y) of row
-// r, line 2r+1 holds (d_z, lap).
-// ---------------------------------------------------------------------------
-template <int L, class G>
-__device__ __forceinline__ void z_c2r_rho_body(
-    const Blk &bk, double2 *lds, const double2 *__restrict__ W, long M,
-    const double *__restrict__ f, double *__restrict__ result,
-    G *__restrict__ grad3, double *__restrict__ rho,
-    double *__restrict__ pressure, double *__restrict__ partials, long nrows,
-    long N, double m2, const double2 *__restrict__ tw, const Ens &e)
+// Line plans of the z pass (512 points: a line in one wavefront)
+template <int L> struct ZRhsPlan { using P = typename ZPlanOf<L>::P; };
+template <> struct ZRhsPlan<32> { using P = PlanT<4, 4, 4, 2>; };
+template <> struct ZRhsPlan<64> { using P = PlanT<4, 4, 4, 4>; };
+template <> struct ZRhsPlan<128> { using P = PlanT<4, 4, 4, 4, 2>; };
+template <> struct ZRhsPlan<256> { using P = PlanT<4, 4, 4, 4, 4>; };
+template <int L> struct ZRhsTile {
+    using P = typename ZRhsPlan<L>::P;
+    static constexpr int E = P::E, T = L / E, PITCH = Lds<L>::PITCH, LPW = 64 / T;
+};
+
+// LDS of the z pass in complex values: the lines, then the stage twiddles
+template <int L, int WG>
+__host__ __device__ constexpr int z_rhs_lines()
 {
-    // realization z of an ensemble
-    W += bk.z * e.w;
-    f += bk.z * e.f;
-    result += bk.z * e.f;
-    partials += bk.z * e.p;
-    if (grad3) grad3 += bk.z * e.g;
-    using TL = Tile<L>;
-    constexpr int MZ = L / 2 + 1;
-    constexpr int RPB = TL::B / 2; // rows per block
-    const int tid = threadIdx.x;
-    const int bc = tid / TL::T;
-    const long line = (long)bk.x * TL::B + bc;
-    const bool act = line < 2 * nrows;
-    const long row = act ? (line >> 1) : 0;
-    const int p = (int)(line & 1);
-    const double2 *A = W + (2 * p) * M + row * MZ;
-    const double2 *Bq = W + (2 * p + 1) * M + row * MZ;
-    // stage twiddles from LDS behind the tile's lines, so that the loads of
-    // phi, dphi, psi below stay in flight through the whole transform
-    tw = twiddles_to_lds_wave<L>(lds + z_rho_lines<L>(), tw);
-    auto rd = [&](int, int n) {
-        const double2 z = herm_merge<L>(A, Bq, n); // in bounds for every lane
-        return act ? z : make_double2(0.0, 0.0);
-    };
-    // Each wavefront finishes the RPW = LPW / 2 rows of its own lines (line
-    // 2 rr holds (d_x, d_y) of row rr, line 2 rr + 1 (d_z, lap)), K = E / 2
-    // points per lane.  phi, dphi, psi of those points are loaded before
-    // the transform, so their latency hides behind it; rows past the end
-    // read row 0 (in bounds, unused)
-    constexpr int RPW = TL::LPW / 2;
-    static_assert(RPW >= 1, "both lines of a row in one wavefront");
-    constexpr int K = RPW * L / 64;
-    static_assert(K * 64 == RPW * L, "whole rows per wavefront sweep");
-    const int w = tid / 64, lane = tid % 64;
-    const long row0 = (long)bk.x * RPB + w * RPW;
-    const double2 *wl = lds + w * TL::LPW * TL::PITCH;
-    double php[K], dphp[K], psp[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        const int idx = lane + k * 64;
-        const int rr = idx / L, n = idx - rr * L;
-        const long r = row0 + rr;
-        const long i = (r < nrows ? r : 0) * L + n;
-        php[k] = f[i];
-        dphp[k] = f[N + i];
-        psp[k] = f[2 * N + i];
+    return WG / ZRhsTile<L>::T * ZRhsTile<L>::PITCH;
+}
+template <int L, int WG>
+__host__ __device__ constexpr int z_rhs_lds()
+{
+    return z_rhs_lines<L, WG>() + L;
+}
+
+// work-groups of the z pass, and its partial sums (one pair a wavefront)
+template <int L>
+inline unsigned z_rhs_blocks(long nrows, int wg)
+{
+    const long lines = wg / ZRhsTile<L>::T;
+    return (unsigned)((nrows / 2 + lines - 1) / lines);
+}
+
+template <class C>
+struct ZRhsArgs {
+    using R = typename CT<C>::R;
+    const double *f;
+    double *result;
+    const double *phi;     // phi, or after the filter phi - *dc
+    const double *dc;      // (NULL: phi itself), rphi and rdc apart
+    const double *gx, *gy; // x and y gradients (k_deriv)
+    R *g3;                 // GW: all three gradients in the source's type
+    C *W;                  // GW: the source components
+    long M, N, Ntot, nrows;
+    double *rho, *pressure; // output calls (else NULL)
+    double *partials;
+    double m2;
+    double k1, k2;         // 2 pi / (L length), (2 pi / length)^2 / L
+    const double2 *tw;
+    const C *twc;          // stage twiddles of the source's type
+    Ens e;
+    long rphi, rdc, rxy, rg, rw; // realization strides of phi, dc, gx / gy, g3, W
+    GwAxis ga;
+};
+
+// source component K of one point from its gradient
+template <int K, class R>
+__device__ __forceinline__ R gw_source(R gx, R gy, R gz, int m)
+{
+    if constexpr (K == 0) {
+        const R q = m == 0 ? gz : gx, d = m == 0 ? gx : (m == 1 ? gy : gz);
+        return q * q - d * d;
+    } else if constexpr (K == 1) {
+        return gx * gy;
+    } else if constexpr (K == 2) {
+        return gx * gz;
+    } else if constexpr (K == 3) {
+        const R q = m == 1 ? gz : gy, d = m == 0 ? gx : (m == 1 ? gy : gz);
+        return q * q - d * d;
+    } else {
+        return gy * gz;
     }
-    fft_line_wave<L, +1, typename TL::P>(lds + bc * TL::PITCH, tid % TL::T, tw, rd);
+}
 
-    const long Ntot = 4 * N + 4 * (2 * M) + 1;
-    const double aa = f[Ntot - 1];
+template <int L, bool GW, class C, int WG>
+__device__ __forceinline__ void z_rhs_body(const Blk &bk, double2 *lds,
+                                           const ZRhsArgs<C> &a)
+{
+    using TL = ZRhsTile<L>;
+    using P = typename TL::P;
+    using R = typename CT<C>::R;
+    constexpr int E = TL::E, T = TL::T, PITCH = TL::PITCH, LPW = TL::LPW;
+    constexpr int NW = WG / 64, MZ = L / 2 + 1;
+    // The other inputs of a point are loaded ahead of the transforms where
+    // too few wavefronts are there to hide their latency (single-wavefront
+    // work-groups: 5.1 against 6.0 us at 32^3; the 64- and 128-point lines of
+    // the GW pass: 137 against 151 us for 16 x 64^3, 278 against 293 for 4 x
+    // 128^3), and at the point elsewhere (256^3 411 against 425 us, 128^3
+    // without GW 24 against 28 us): the registers cost a wave a SIMD.
+    constexpr bool PRE = WG == 64 || (GW && (L == 64 || L == 128));
+    const int w = (int)threadIdx.x / 64, lane = (int)threadIdx.x % 64;
+    const int j = lane % T;
+    const long wave = (long)bk.x * NW + w, line0 = wave * LPW;
+    const long line = line0 + lane / T;
+    const bool act = line < a.nrows / 2; // idle lanes work on line 0
+    const long ia = (act ? 2 * line : 0) * L; // row A; row B is L further
+    double2 *wl = lds + w * LPW * PITCH, *my = wl + lane / T * PITCH;
+    const double2 *tw = twiddles_to_lds_wave<L>(lds + z_rhs_lines<L, WG>(), a.tw);
+    const double *__restrict__ f = a.f + bk.z * a.e.f;
+    const double *__restrict__ lx = a.result + bk.z * a.e.f + a.N;
+    const double *__restrict__ ly = lx + a.N;
+    const double *__restrict__ gxp = a.gx + bk.z * a.rxy;
+    const double *__restrict__ gyp = a.gy + bk.z * a.rxy;
+    double *__restrict__ outA = a.result + bk.z * a.e.f;
+    double *__restrict__ outp = outA + 3 * a.N;
+
+    // the derivatives of phi - phi[0] (see deriv_body)
+    const double *__restrict__ phi = a.phi + bk.z * a.rphi;
+    const double phi0 = phi[0];
+    const double dc = a.dc ? a.dc[bk.z * a.rdc] : 0.0;
+    double2 ph[E], lz[E], dz[E];
+#pragma unroll
+    for (int s = 0; s < E; ++s) {
+        const long i = ia + stage1_point<L, P>(j, s);
+        ph[s] = make_double2(phi[i], phi[i + L]);
+    }
+    // the other inputs of the points this thread ends with (rows A and B)
+    struct In {
+        double2 lx, ly, gx, gy, dph, ps;
+    };
+    auto load = [&](int s) {
+        const long i = ia + last_point<L, P>(j, s);
+        return In{make_double2(lx[i], lx[i + L]), make_double2(ly[i], ly[i + L]),
+                  make_double2(gxp[i], gxp[i + L]), make_double2(gyp[i], gyp[i + L]),
+                  make_double2(f[a.N + i], f[a.N + i + L]),
+                  make_double2(f[2 * a.N + i], f[2 * a.N + i + L])};
+    };
+    In in[PRE ? E : 1];
+    if constexpr (PRE) {
+#pragma unroll
+        for (int s = 0; s < E; ++s) in[s] = load(s);
+    }
+    {
+        double2 spec[E];
+        fft_line_wave_regs<L, -1, P>(
+            my, j, tw,
+            [&](int s, int) {
+                return make_double2(ph[s].x - phi0, ph[s].y - phi0);
+            },
+            [&](int s, int, double2 v) { spec[s] = v; });
+        line_sync<true>();
+        fft_line_wave_regs<L, +1, P>(
+            my, j, tw,
+            [&](int s, int n) {
+                const double2 v = spec[chain_slot<L, P>(s)];
+                const double m = n > L / 2 ? L - n : n, k = -(a.k2 * m * m);
+                return make_double2(v.x * k, v.y * k);
+            },
+            [&](int s, int, double2 v) { lz[s] = v; });
+        line_sync<true>();
+        fft_line_wave_regs<L, +1, P>(
+            my, j, tw,
+            [&](int s, int n) {
+                const double2 v = spec[chain_slot<L, P>(s)];
+                const double k = n > L / 2 ? a.k1 * (n - L)
+                                           : (2 * n == L ? 0.0 : a.k1 * n);
+                return make_double2(-v.y * k, v.x * k);
+            },
+            [&](int s, int, double2 v) { dz[s] = v; });
+    }
+    const double aa = f[a.Ntot - 1];
     const double a2 = aa * aa;
     double srho = 0.0, sp = 0.0;
+    [[maybe_unused]] C gx[E], gy[E], gz[E];
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-        const int idx = lane + k * 64;
-        const int rr = idx / L, n = idx - rr * L;
-        const long r = row0 + rr;
-        if (r >= nrows) continue;
-        const double2 z1 = wl[(2 * rr) * TL::PITCH + Lds<L>::idx(n)];
-        const double2 z2 = wl[(2 * rr + 1) * TL::PITCH + Lds<L>::idx(n)];
-        const double dx = z1.x, dy = z1.y, dz = z2.x, lap = z2.y;
-        double g = dx * dx;
-        g += dy * dy;
-        g += dz * dz;
-        const long i = r * L + n;
-        const double ph = php[k], dph = dphp[k], ps = psp[k];
-        const double t1 = (0.5 - ps) * dph * dph;
-        const double t2 = (0.5 + ps) * g / a2;
-        const double V = m2 * ph * ph / 2.0;
-        const double rv = t1 + t2 + V;
-        const double pv = t1 - t2 / 3.0 - V;
-        result[N + i] = lap;
-        result[3 * N + i] = pv;
-        if (grad3) {
-            grad3[i] = (G)dx;
-            grad3[N + i] = (G)dy;
-            grad3[2 * N + i] = (G)dz;
+    for (int s = 0; s < E; ++s) {
+        const long i = ia + last_point<L, P>(j, s);
+        const double2 p = ph[unchain_slot<L, P>(s)];
+        if constexpr (!PRE) in[0] = load(s);
+        const In &v = in[PRE ? s : 0];
+        auto point = [&](long q, double p0, double d_x, double d_y, double d_z,
+                         double lap, double dph, double ps) {
+            double g = d_x * d_x;
+            g += d_y * d_y;
+            g += d_z * d_z;
+            const double t1 = (0.5 - ps) * dph * dph;
+            const double t2 = (0.5 + ps) * g / a2;
+            const double V = a.m2 * p0 * p0 / 2.0;
+            const double rv = t1 + t2 + V;
+            const double pv = t1 - t2 / 3.0 - V;
+            const double A = (1.0 + 4.0 * ps) * lap / a2 -
+                             (1.0 + 2.0 * ps) * (a.m2 * p0);
+            if (act) {
+                outA[q] = A;
+                outp[q] = pv;
+                if (a.rho) {
+                    a.rho[q] = rv;
+                    a.pressure[q] = pv;
+                }
+                if constexpr (GW) {
+                    R *g3 = a.g3 + bk.z * a.rg;
+                    if constexpr (sizeof(R) == 4) {
+                        g3[q] = (R)d_x;
+                        g3[a.N + q] = (R)d_y;
+                    }
+                    g3[2 * a.N + q] = (R)d_z;
+                }
+                srho += rv;
+                sp += pv;
+            }
+        };
+        point(i, p.x + dc, v.gx.x, v.gy.x, dz[s].x, v.lx.x + v.ly.x + lz[s].x,
+              v.dph.x, v.ps.x);
+        point(i + L, p.y + dc, v.gx.y, v.gy.y, dz[s].y, v.lx.y + v.ly.y + lz[s].y,
+              v.dph.y, v.ps.y);
+        if constexpr (GW) {
+            gx[s] = CT<C>::make((R)v.gx.x, (R)v.gx.y);
+            gy[s] = CT<C>::make((R)v.gy.x, (R)v.gy.y);
+            gz[s] = CT<C>::make((R)dz[s].x, (R)dz[s].y);
         }
-        if (rho) {
-            rho[i] = rv;
-            pressure[i] = pv;
-        }
-        srho += rv;
-        sp += pv;
     }
-    double *sh = reinterpret_cast<double *>(lds);
-    srho = block_reduce<OpSum>(srho, sh, FFT_WG);
-    sp = block_reduce<OpSum>(sp, sh + 8, FFT_WG);
-    if (tid == 0) {
-        partials[2 * bk.x] = srho;
-        partials[2 * bk.x + 1] = sp;
+    srho = wave_reduce<OpSum>(srho);
+    sp = wave_reduce<OpSum>(sp);
+    if (lane == 0) {
+        double *part = a.partials + bk.z * a.e.p + 2 * wave;
+        part[0] = srho;
+        part[1] = sp;
+    }
+    if constexpr (GW) {
+        C *const cl = reinterpret_cast<C *>(wl); // the wavefront's own lines
+        C *const cmy = cl + lane / T * PITCH;
+        const long row0 = 2 * line0;
+        C *const Wo = a.W + bk.z * a.rw + row0 * MZ;
+        // FP64: the LDS table; FP32: its own in global memory
+        const C *twc;
+        if constexpr (sizeof(R) == 8)
+            twc = tw;
+        else
+            twc = a.twc;
+        auto comp = [&](auto kc) {
+            constexpr int K = decltype(kc)::value;
+            line_sync<true>(); // earlier LDS reads of these lines are done
+            fft_line_impl<L, -1, true, false, P, C, true>(
+                cmy, cmy, j, twc,
+                [&](int s, int) {
+                    const int q = chain_slot<L, P>(s);
+                    return CT<C>::make(gw_source<K>(gx[q].x, gy[q].x, gz[q].x, a.ga.m),
+                                       gw_source<K>(gx[q].y, gy[q].y, gz[q].y, a.ga.m));
+                },
+                NoWrite());
+            for (int idx = lane; idx < 2 * LPW * MZ; idx += 64) {
+                const int r = idx / MZ, k = idx - r * MZ;
+                if (row0 + r < a.nrows)
+                    Wo[K * a.M + idx] = herm_split<L>(cl + (r >> 1) * PITCH, k, r & 1);
+            }
+        };
+        comp(std::integral_constant<int, 0>{});
+        comp(std::integral_constant<int, 1>{});
+        comp(std::integral_constant<int, 2>{});
+        comp(std::integral_constant<int, 3>{});
+        comp(std::integral_constant<int, 4>{});
     }
 }
 
-template <int L, class G>
-__global__ __launch_bounds__(FFT_WG) void k_z_c2r_rho(
-    const double2 *__restrict__ W, long M, const double *__restrict__ f,
-    double *__restrict__ result, G *__restrict__ grad3,
-    double *__restrict__ rho, double *__restrict__ pressure,
-    double *__restrict__ partials, long nrows, long N, double m2,
-    const double2 *__restrict__ tw, Ens e)
+template <int L, bool GW, class C, int WG>
+__global__ __launch_bounds__(WG) void k_z_rhs(ZRhsArgs<C> a)
 {
-    __shared__ double2 lds[z_rho_lds<L>()];
-    z_c2r_rho_body<L, G>(hw_blk(), lds, W, M, f, result, grad3, rho, pressure,
-                         partials, nrows, N, m2, tw, e);
+    __shared__ double2 lds[z_rhs_lds<L, WG>()];
+    z_rhs_body<L, GW, C, WG>(hw_blk(), lds, a);
+}
+
+// The derivative passes of nr realizations of a context: the field they
+// differentiate (phi of f, or after the filter the fluctuations that the
+// filter's last pass kept) and where the x and y gradients go
+struct DerivIO {
+    const double *phi;
+    const double *dc;
+    double *gx, *gy;
+    long rphi, rdc, rxy; // realization strides (doubles)
+};
+DerivIO deriv_io(const ihg_ctx *c, const double *f, int filtered, int nr);
+DerivXY deriv_axes(const ihg_ctx *c, const DerivIO &io, double *result, int nr);
+
+// the filter's round trip and last pass
+FilterFac filter_fac(const ihg_ctx *c, int output, int nr);
+ZShift filter_shift(const ihg_ctx *c, int nr);
+
+// the z pass of nr realizations of a context (no output arrays)
+template <class C>
+inline ZRhsArgs<C> z_rhs_args(const ihg_ctx *c, const double *f,
+                              double *result, const DerivIO &io, int nr)
+{
+    using R = typename CT<C>::R;
+    ZRhsArgs<C> a{};
+    a.f = f;
+    a.result = result;
+    a.phi = io.phi;
+    a.dc = io.dc;
+    a.gx = io.gx;
+    a.gy = io.gy;
+    a.rphi = io.rphi;
+    a.rdc = io.rdc;
+    a.rxy = io.rxy;
+    a.g3 = reinterpret_cast<R *>(c->grad3);
+    a.W = reinterpret_cast<C *>(c->W);
+    a.M = c->M;
+    a.N = c->N;
+    a.Ntot = c->Ntot;
+    a.nrows = (long)c->Nx * c->Ny;
+    a.partials = c->partials;
+    a.m2 = c->p.mass * c->p.mass;
+    a.k1 = c->kg.kz1 / c->Nz;
+    a.k2 = c->kg.kz2 / c->Nz;
+    a.ga = gw_axis(c->kg);
+    a.tw = c->tw;
+    if constexpr (sizeof(R) == 4)
+        a.twc = c->twf;
+    else
+        a.twc = c->tw;
+    if (nr > 1) {
+        a.e = c->ens;
+        a.rg = c->ens.g;
+        a.rw = c->ens.w * (long)(sizeof(double2) / sizeof(C));
+    }
+    return a;
 }
 
 // rho_mean, pressure_mean (src/toolbox.c:241-242) and da (src/toolbox.c:87)
-// (one work-group per realization r; sh: 8 doubles of LDS)
+// (one work-group per realization r; sh: MEANS_WG / 64 doubles of LDS)
 // EP: the RK4 epilogue of the scale factor's slope
+constexpr int MEANS_WG = 1024;
 template <bool EP = false>
 __device__ __forceinline__ void means_body(
     unsigned r, double *sh, const double *__restrict__ partials, int nparts,
@@ -224,13 +444,13 @@ __device__ __forceinline__ void means_body(
     const double2 *p2 = reinterpret_cast<const double2 *>(partials);
     double s0 = 0.0, s1 = 0.0;
 #pragma unroll 4
-    for (int i = threadIdx.x; i < nparts; i += RED_WG) {
+    for (int i = threadIdx.x; i < nparts; i += MEANS_WG) {
         const double2 v = p2[i];
         s0 += v.x;
         s1 += v.y;
     }
-    s0 = block_reduce<OpSum>(s0, sh, RED_WG);
-    s1 = block_reduce<OpSum>(s1, sh, RED_WG);
+    s0 = block_reduce<OpSum>(s0, sh, MEANS_WG);
+    s1 = block_reduce<OpSum>(s1, sh, MEANS_WG);
     if (threadIdx.x == 0) {
         const double rm = s0 / N, pm = s1 / N;
         dscal[S_RHO_MEAN] = rm;
@@ -243,22 +463,20 @@ __device__ __forceinline__ void means_body(
     }
 }
 
-// update_phi_psi (src/toolbox.c:282-299); lap and p were parked in
-// result[N..2N) and result[3N..4N) by k_z_c2r_rho
+// update_phi_psi (src/toolbox.c:282-299); the part A of the slope of dphi and
+// p were parked in result[0..N) and result[3N..4N) by k_z_rhs
 // (work-group bx of gx on realization z; EP: the RK4 epilogue of the four
 // blocks' slopes)
 template <bool NT, bool EP = false>
 __device__ __forceinline__ void update_phi_psi_body(
     unsigned bx, unsigned gx, unsigned z, const double *__restrict__ f,
-    double *__restrict__ result, long N, long Ntot, double m2,
+    double *__restrict__ result, long N,
     const double *__restrict__ dscal, const Ens &e, const Rk4Ep &ep0 = Rk4Ep{})
 {
     f += z * e.f;
     result += z * e.f;
     dscal += z * e.s;
     [[maybe_unused]] const Rk4Ep ep = EP ? ep0.shifted(z * e.f) : ep0;
-    const double aa = f[Ntot - 1];
-    const double a2 = aa * aa;
     const double hubble = sqrt(dscal[S_RHO_MEAN] / 3.0);
     const double h3 = 3.0 * hubble;
     const double pm = dscal[S_P_MEAN];
@@ -269,14 +487,11 @@ __device__ __forceinline__ void update_phi_psi_body(
     double2 *Rs = reinterpret_cast<double2 *>(result);
     const long H = N / 2;
     for (long i = (long)bx * RED_WG + threadIdx.x; i < H; i += stride) {
-        const double2 ph = ld2<NT>(F + i), dph = ld2<NT>(F + H + i),
-                      ps = ld2<NT>(F + 2 * H + i), dps = ld2<NT>(F + 3 * H + i);
-        const double2 lap = ld2<NT>(Rs + H + i), pr = ld2<NT>(Rs + 3 * H + i);
-        const double2 r1 = make_double2(
-            (1.0 + 4.0 * ps.x) * lap.x / a2 - (h3 - 4.0 * dps.x) * dph.x -
-                (1.0 + 2.0 * ps.x) * (m2 * ph.x),
-            (1.0 + 4.0 * ps.y) * lap.y / a2 - (h3 - 4.0 * dps.y) * dph.y -
-                (1.0 + 2.0 * ps.y) * (m2 * ph.y));
+        const double2 dph = ld2<NT>(F + H + i), ps = ld2<NT>(F + 2 * H + i),
+                      dps = ld2<NT>(F + 3 * H + i);
+        const double2 A = ld2<NT>(Rs + i), pr = ld2<NT>(Rs + 3 * H + i);
+        const double2 r1 = make_double2(A.x - (h3 - 4.0 * dps.x) * dph.x,
+                                        A.y - (h3 - 4.0 * dps.y) * dph.y);
         const double2 r3 = make_double2(
             0.5 * pr.x + (ps.x - 0.5) * pm - 4.0 * hubble * dps.x,
             0.5 * pr.y + (ps.y - 0.5) * pm - 4.0 * hubble * dps.y);
@@ -297,113 +512,10 @@ __device__ __forceinline__ void update_phi_psi_body(
 template <bool NT>
 __global__ __launch_bounds__(RED_WG) void k_update_phi_psi(
     const double *__restrict__ f, double *__restrict__ result, long N,
-    long Ntot, double m2, const double *__restrict__ dscal, Ens e)
+    const double *__restrict__ dscal, Ens e)
 {
     update_phi_psi_body<NT>(blockIdx.x, gridDim.x, blockIdx.z, f, result, N,
-                            Ntot, m2, dscal, e);
-}
-
-// ---------------------------------------------------------------------------
-// GW sources: z r2c of the products d_i phi d_j phi (mk_gw_sources,
-// src/toolbox.c:410-424).  Only the transverse traceless part of the source
-// enters the equations, and the projection takes delta_ij s to 0 for every s
-// (P is a projector of trace 2 built from the full k with k_i k_i = k^2), so
-// d_z phi d_z phi is subtracted from the diagonal: five components (xx - zz,
-// xy, xz, yy - zz, yz) are transformed instead of six.  That takes a sixth
-// off the transforms of the source (two DOPRI853 steps at 256^3 86.0 -> 83.9
-// ms, 5 RK4 steps of 48 x 32^3 + 16 x 64^3 + 4 x 128^3 50.6 -> 49.0 ms); the
-// error of the slopes of h against 64-bit torch is what it was with six
-// (8e-16 to 1.5e-15 of the source alone, 4^3 to 512-point lines).
-// A work-group owns B rows: every thread loads its first-stage points of
-// d_x phi, d_y phi, d_z phi once into registers, then the complex rows (xx -
-// zz, xy), (xz, yy - zz), (yz, 0) of each row are transformed one after the
-// other; component c = 2q + s goes to W + c M.
-// ---------------------------------------------------------------------------
-constexpr int GW_NC = 5;
-
-template <int L, int Q, class C, class Rows>
-__device__ __forceinline__ void sources_pair(C *lds, int tid, const Rows &g,
-                                             bool act, C *__restrict__ W,
-                                             long M, long row0, long nrows,
-                                             const C *__restrict__ tw)
-{
-    using TL = Tile<L>;
-    using R = typename CT<C>::R;
-    constexpr int MZ = L / 2 + 1;
-    const int bc = tid / TL::T;
-    auto rd = [&](int s, int) {
-        R u, v;
-        if constexpr (Q == 0) {
-            u = g.x[s] * g.x[s] - g.z[s] * g.z[s];
-            v = g.x[s] * g.y[s];
-        } else if constexpr (Q == 1) {
-            u = g.x[s] * g.z[s];
-            v = g.y[s] * g.y[s] - g.z[s] * g.z[s];
-        } else {
-            u = g.y[s] * g.z[s];
-            v = 0;
-        }
-        return act ? CT<C>::make(u, v) : CT<C>::make(0, 0);
-    };
-    fft_line_wave<L, -1, typename TL::P>(lds + bc * TL::PITCH, tid % TL::T, tw, rd);
-    // each wavefront splits and stores the rows of its own lines
-    constexpr int NS = Q == 2 ? 1 : 2; // components of the pair
-    const int w = tid / 64, lane = tid % 64;
-    for (int idx = lane; idx < TL::LPW * NS * MZ; idx += 64) {
-        const int lb = w * TL::LPW + idx / (NS * MZ);
-        const int rem = idx - (lb - w * TL::LPW) * NS * MZ;
-        const int s = rem / MZ, k = rem - s * MZ;
-        const long r = row0 + lb;
-        if (r < nrows)
-            W[(2 * Q + s) * M + r * MZ + k] =
-                herm_split<L>(lds + lb * TL::PITCH, k, s);
-    }
-    line_sync<true>(); // split reads done before the next transform
-}
-
-template <int L, class R>
-struct GradRegs {
-    R x[Tile<L>::E], y[Tile<L>::E], z[Tile<L>::E];
-};
-
-// C = double2: the FP64 path; C = float2: the precision form (gradients
-// stored in FP32, products, FFTs and output in FP32)
-template <int L, class C>
-__device__ __forceinline__ void z_r2c_sources_body(
-    const Blk &bk, C *lds, const typename CT<C>::R *__restrict__ g3,
-    C *__restrict__ W, long M, long nrows, long N, const C *__restrict__ tw,
-    long rg, long rw)
-{
-    g3 += bk.z * rg;
-    W += bk.z * rw;
-    using TL = Tile<L>;
-    using R = typename CT<C>::R;
-    const int tid = threadIdx.x;
-    const int bc = tid / TL::T, j = tid % TL::T;
-    const long row0 = (long)bk.x * TL::B;
-    const long row = row0 + bc;
-    const bool act = row < nrows;
-    const R *gx = g3 + (act ? row : 0) * L;
-    GradRegs<L, R> g;
-#pragma unroll
-    for (int s = 0; s < TL::E; ++s) {
-        const int n = stage1_point<L, typename TL::P>(j, s);
-        g.x[s] = gx[n];
-        g.y[s] = gx[N + n];
-        g.z[s] = gx[2 * N + n];
-    }
-    sources_pair<L, 0>(lds, tid, g, act, W, M, row0, nrows, tw);
-    sources_pair<L, 1>(lds, tid, g, act, W, M, row0, nrows, tw);
-    sources_pair<L, 2>(lds, tid, g, act, W, M, row0, nrows, tw);
-}
-
-template <int L, class C>
-__global__ __launch_bounds__(FFT_WG) void k_z_r2c_sources(
-    const typename CT<C>::R *__restrict__ g3, C *__restrict__ W, long M,
-    long nrows, long N, const C *__restrict__ tw, long rg, long rw)
-{
-    __shared__ C lds[Tile<L>::B * Tile<L>::PITCH];
-    z_r2c_sources_body<L, C>(hw_blk(), lds, g3, W, M, nrows, N, tw, rg, rw);
+                            dscal, e);
 }
 
 // ---------------------------------------------------------------------------
@@ -415,8 +527,10 @@ __global__ __launch_bounds__(FFT_WG) void k_z_r2c_sources(
 //   o0 = S_pp - 2 f_p (sum_j k_j S_pj) + (f_p k_p s1 + s2) / 2
 //   o1 = S_pq - f_p (sum_j k_j S_qj) - f_q (sum_j k_j S_pj) + f_p k_q s1 / 2
 // alpha_C, beta_C are the derivatives of these with respect to component
-// C = 0..4 = (xx, xy, xz, yy, yz) (zz is subtracted from the diagonal); the
-// k = 0 mode projects to 0.
+// C = 0..5 = (xx, xy, xz, yy, yz, zz); the k = 0 mode projects to 0.
+// tt_source_coef<K> gives those of source component K: zz in the place of xx
+// (K = 0) where xx is the product subtracted from the others, of yy (K = 3)
+// where yy is.
 // ---------------------------------------------------------------------------
 template <int C, class R>
 __device__ __forceinline__ void tt_coef(R kx, R ky, R kz, R inv_ksq,
@@ -442,14 +556,31 @@ __device__ __forceinline__ void tt_coef(R kx, R ky, R kz, R inv_ksq,
     } else if constexpr (C == 3) {
         t1 = ky * fy; t2 = I; rowp = py ? ky : O; rowq = qy ? ky : O;
         dpp = py ? I : O; dpq = O;
-    } else {
+    } else if constexpr (C == 4) {
         t1 = D * (ky * fz); t2 = O; rowp = py ? kz : O;
         rowq = qy ? kz : ky; dpp = O; dpq = py ? I : O;
+    } else {
+        t1 = kz * fz; t2 = I; rowp = O; rowq = qy ? O : kz;
+        dpp = O; dpq = O;
     }
     const R s1 = t1 + t2, s2 = t1 - t2;
     const R half = (R)0.5, two = (R)2.0;
     al = zero ? (R)0 : dpp - two * fp * rowp + half * (fp * kp * s1 + s2);
     be = zero ? (R)0 : dpq - fp * rowq - fq * rowp + half * fp * kq * s1;
+}
+
+template <int K, class R>
+__device__ __forceinline__ void tt_source_coef(R kx, R ky, R kz, R inv_ksq,
+                                               bool b1, bool zero, int m,
+                                               R &al, R &be)
+{
+    if constexpr (K == 0 || K == 3) {
+        if (m == (K == 0 ? 0 : 1)) { // uniform
+            tt_coef<5>(kx, ky, kz, inv_ksq, b1, zero, al, be);
+            return;
+        }
+    }
+    tt_coef<K>(kx, ky, kz, inv_ksq, b1, zero, al, be);
 }
 
 // y transform of source component K (its z and x passes are done) with the
@@ -462,12 +593,12 @@ __device__ __forceinline__ void tt_coef(R kx, R ky, R kz, R inv_ksq,
 // exchanges.  Components alternate between two LDS buffers: the barrier of
 // component K also ends every wavefront's use of the buffer component K + 1
 // writes.  kx, kz, b1 (|k_z| > eps) and z0 (ix = iz = 0) are those of line
-// lw, inv_ksq the 1/k^2 of its points.
+// lw, inv_ksq the 1/k^2 of its points, m the axis of GwAxis.
 template <int L, class P, int K, class C>
 __device__ __forceinline__ void tt_component(
     C *lb, C *lw, int j, int jw, const C *__restrict__ tw, const C *cur,
     const KGeom &kg, typename CT<C>::R kx, typename CT<C>::R kz, bool b1,
-    bool z0, const typename CT<C>::R *inv_ksq, C *o0, C *o1)
+    bool z0, const typename CT<C>::R *inv_ksq, int m, C *o0, C *o1)
 {
     using R = typename CT<C>::R;
     // Register pressure control (empty asm statements, no instructions):
@@ -491,7 +622,7 @@ __device__ __forceinline__ void tt_component(
         asm volatile("" : "+v"(iv));
         const bool zero = z0 && (n == 0);
         R al, be;
-        tt_coef<K>(kx, (R)kg.kyf(n), kz, iv, b1, zero, al, be);
+        tt_source_coef<K>(kx, (R)kg.kyf(n), kz, iv, b1, zero, m, al, be);
         if constexpr (K == 0) {
             o0[s] = CT<C>::make(al * v.x, al * v.y);
             o1[s] = CT<C>::make(be * v.x, be * v.y);
@@ -537,7 +668,8 @@ __device__ __forceinline__ void y_tt_update_h_body(
     const Blk &bk, C *lds, const C *W, long M, const double *__restrict__ f,
     double *__restrict__ result, long N, long Next, long Ntot,
     const KGeom &kg, const double *__restrict__ dscal, const LineSet &ls,
-    const C *__restrict__ tw, const Ens &e, long rw, const Rk4Ep &ep0 = Rk4Ep{})
+    const C *__restrict__ tw, const Ens &e, long rw, GwAxis ga,
+    const Rk4Ep &ep0 = Rk4Ep{})
 {
     // realization z of an ensemble (rw: its W stride in units of C)
     W += bk.z * rw;
@@ -625,8 +757,8 @@ __device__ __forceinline__ void y_tt_update_h_body(
         constexpr int K = decltype(kc)::value;
         if constexpr (K == GW_NC - 1 && EARLY) load_h();
         tt_component<L, P, K>(K % 2 ? lb1 : lb0, K % 2 ? lw1 : lw0, j, jw, tw,
-                              bufs[K % 2], kg, kxw, kzw, b1w, z0w, inv, o0,
-                              o1);
+                              bufs[K % 2], kg, kxw, kzw, b1w, z0w, inv, ga.m,
+                              o0, o1);
         if constexpr (K + 2 < GW_NC) load(K + 2, bufs[K % 2]);
     };
     step(std::integral_constant<int, 0>{});
@@ -695,11 +827,11 @@ __global__ __launch_bounds__(WG) void k_y_tt_update_h(
     const C *W, long M, const double *__restrict__ f,
     double *__restrict__ result, long N, long Next, long Ntot, KGeom kg,
     const double *__restrict__ dscal, LineSet ls, const C *__restrict__ tw,
-    Ens e, long rw)
+    Ens e, long rw, GwAxis ga)
 {
     __shared__ C lds[tt_lds<L, WG, P>()];
     y_tt_update_h_body<L, WG, P, C>(hw_blk(), lds, W, M, f, result, N, Next,
-                                    Ntot, kg, dscal, ls, tw, e, rw);
+                                    Ntot, kg, dscal, ls, tw, e, rw, ga);
 }
 
 

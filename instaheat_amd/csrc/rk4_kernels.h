@@ -11,10 +11,12 @@
 
 namespace ihg {
 
-// one element of a stage: y + dt k / 2 (half) or y + dt k
+// one element of a stage: y + dt k / 2 (half) or y + dt k (multiply-adds
+// fused within the expression only, so that every unit computes the same)
 __device__ __forceinline__ double rk4_stage_val(double y, double k, double dt,
                                                 int half)
 {
+#pragma clang fp contract(on)
     return half ? y + dt * k / 2.0 : y + dt * k;
 }
 
@@ -22,6 +24,7 @@ __device__ __forceinline__ double rk4_stage_val(double y, double k, double dt,
 __device__ __forceinline__ double rk4_final_val(double y, double k1, double k2,
                                                 double k3, double k4, double dt)
 {
+#pragma clang fp contract(on)
     return y + dt * (k1 + 2.0 * k2 + 2.0 * k3 + k4) / 6.0;
 }
 
