@@ -80,7 +80,7 @@ constexpr int fam_lds_max()
                      Fam::template lds<64>(), Fam::template lds<128>()});
 }
 
-// LDS of the strided and derivative bodies: none for one-stage plans, whose
+// LDS of the strided bodies: none for one-stage plans, whose
 // only stage loads from and stores to registers
 template <int L>
 constexpr int strided_lds()
@@ -238,7 +238,11 @@ struct FamDeriv {
         DerivAxis a;
         const double2 *tw;
     };
-    template <int L> static constexpr int lds() { return strided_lds<L>(); }
+    template <int L>
+    static constexpr int lds()
+    {
+        return StridedShape<L, typename DerivPlan<L>::P, WG>::LDS;
+    }
     template <int L>
     __device__ static void run(const Blk &bk, double2 *lds, const Args &a)
     {
@@ -303,11 +307,11 @@ struct FamUpdate {
     __device__ static void run(const Blk &bk, double2 *, const Args &a)
     {
         if (a.nt)
-            update_phi_psi_body<true, EP>(bk.x, bk.gx, bk.z, a.f, a.result, a.N,
-                                          a.dscal, a.e, a.ep);
+            update_after_means_body<true, EP>(bk.x, bk.gx, bk.z, a.f, a.result,
+                                              a.N, a.dscal, a.e, a.ep);
         else
-            update_phi_psi_body<false, EP>(bk.x, bk.gx, bk.z, a.f, a.result,
-                                           a.N, a.dscal, a.e, a.ep);
+            update_after_means_body<false, EP>(bk.x, bk.gx, bk.z, a.f, a.result,
+                                               a.N, a.dscal, a.e, a.ep);
     }
 };
 

@@ -43,7 +43,7 @@ __global__ __launch_bounds__(MEANS_WG) void k_means(
     means_body(blockIdx.x, sh, partials, nparts, N, f, result, Ntot, dscal, e);
 }
 
-// the same three kernels with the RK4 epilogue of their slopes
+// (with the RK4 epilogue of the scale factor's slope)
 __global__ __launch_bounds__(MEANS_WG) void k_means_rk4(
     const double *__restrict__ partials, int nparts, long N,
     const double *__restrict__ f, double *__restrict__ result, long Ntot,
@@ -55,12 +55,41 @@ __global__ __launch_bounds__(MEANS_WG) void k_means_rk4(
 }
 
 template <bool NT>
+__global__ __launch_bounds__(RED_WG) void k_update_phi_psi(
+    const double *__restrict__ f, double *__restrict__ result, long N,
+    const double *__restrict__ dscal, Ens e)
+{
+    update_after_means_body<NT>(blockIdx.x, gridDim.x, blockIdx.z, f, result, N,
+                                dscal, e);
+}
+
+template <bool NT>
 __global__ __launch_bounds__(RED_WG) void k_update_phi_psi_rk4(
     const double *__restrict__ f, double *__restrict__ result, long N,
     const double *__restrict__ dscal, Ens e, Rk4Ep ep)
 {
-    update_phi_psi_body<NT, true>(blockIdx.x, gridDim.x, blockIdx.z, f, result,
-                                  N, dscal, e, ep);
+    update_after_means_body<NT, true>(blockIdx.x, gridDim.x, blockIdx.z, f,
+                                      result, N, dscal, e, ep);
+}
+
+// k_means and the update in one launch for few partial sums: every
+// work-group adds them up itself (the same sums bit for bit), the first of a
+// realization also stores the means and does the scale factor.
+template <bool EP>
+__global__ __launch_bounds__(RED_WG) void k_means_update(
+    const double *__restrict__ partials, int nparts, long N,
+    const double *__restrict__ f, double *__restrict__ result, long Ntot,
+    double *__restrict__ dscal, Ens e, Rk4Ep ep)
+{
+    __shared__ double sh[2 * MEANS_WG / 64];
+    const unsigned z = blockIdx.z;
+    double s0, s1;
+    means_sums(partials + z * e.p, nparts, sh, s0, s1);
+    const double rm = s0 / N, pm = s1 / N;
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        means_store<EP>(z, rm, pm, f, result, Ntot, dscal, e, ep);
+    update_phi_psi_body<false, EP>(blockIdx.x, gridDim.x, z, f, result, N, rm,
+                                   pm, e, ep);
 }
 
 template <int L, int WG, class P>
@@ -261,6 +290,25 @@ int rhs_core(ihg_ctx *c, double *f, double *result, int output, int filtered,
         IHG_TRY(z_pass<float2>(c, f, result, output, io, nr, nparts));
     else
         IHG_TRY(z_pass<double2>(c, f, result, output, io, nr, nparts));
+    // the epilogue reads y (and k1..k3) and writes the stage output beside
+    // the slope: 2 (stage) or 4 (final, no slope written) more blocks
+    const double ep_blocks = !ep ? 0.0 : (ep->mode == RK4_FINAL ? 4.0 : 8.0);
+    const dim3 ugrid(nblocks(N, RED_WG * 4, 65536), 1, nr);
+    // One launch where the partial sums are few (64^3 has 512): 4.6 us against
+    // 3.6 + 3.0 at 16^3, 6.3 against 4.4 + 5.2 at 64^3; every work-group then
+    // reads all of them (at most 16 KB, from L2).
+    if (nparts <= MEANS_WG && 4.0 * 8.0 * (double)N * nr < NT_BYTES)
+        return timed(c, F_UPDATE, (9.0 + ep_blocks) * 8.0 * N * nr, [&]() {
+            if (ep)
+                hipLaunchKernelGGL(k_means_update<true>, ugrid, dim3(RED_WG), 0,
+                                   c->stream, c->partials, nparts, N, f, result,
+                                   c->Ntot, c->dscal, e, *ep);
+            else
+                hipLaunchKernelGGL(k_means_update<false>, ugrid, dim3(RED_WG), 0,
+                                   c->stream, c->partials, nparts, N, f, result,
+                                   c->Ntot, c->dscal, e, Rk4Ep{});
+            return hip_check(hipGetLastError(), "k_means_update");
+        });
     IHG_TRY(timed(c, F_MEANS, 16.0 * nparts * nr, [&]() {
         if (ep)
             hipLaunchKernelGGL(k_means_rk4, dim3(nr), dim3(MEANS_WG), 0,
@@ -272,26 +320,31 @@ int rhs_core(ihg_ctx *c, double *f, double *result, int output, int filtered,
                                c->dscal, e);
         return hip_check(hipGetLastError(), "k_means");
     }));
-    // the epilogue reads y (and k1..k3) and writes the stage output beside
-    // the slope: 2 (stage) or 4 (final, no slope written) more blocks
-    const double ep_blocks = !ep ? 0.0 : (ep->mode == RK4_FINAL ? 4.0 : 8.0);
     return timed(c, F_UPDATE, (9.0 + ep_blocks) * 8.0 * N * nr, [&]() {
         // the streaming hint when the four blocks of all realizations
         // outgrow the caches
         const bool nt = 4.0 * 8.0 * (double)N * nr >= NT_BYTES;
-        const dim3 grid(nblocks(N, RED_WG * 4, 65536), 1, nr);
         if (ep)
             hipLaunchKernelGGL((nt ? k_update_phi_psi_rk4<true>
                                    : k_update_phi_psi_rk4<false>),
-                               grid, dim3(RED_WG), 0, c->stream, f, result, N,
+                               ugrid, dim3(RED_WG), 0, c->stream, f, result, N,
                                c->dscal, e, *ep);
         else
             hipLaunchKernelGGL((nt ? k_update_phi_psi<true>
                                    : k_update_phi_psi<false>),
-                               grid, dim3(RED_WG), 0, c->stream, f, result, N,
+                               ugrid, dim3(RED_WG), 0, c->stream, f, result, N,
                                c->dscal, e);
         return hip_check(hipGetLastError(), "k_update_phi_psi");
     });
+}
+
+// Whether the TT pass transforms the components side by side: up to about two
+// 64^3 grids.  Measured side by side and in turn: 7 x 16^3 6.2 and 13.3 us, 3
+// x 32^3 7.4 and 16.3, 64^3 (135 k modes) 12.0 and 13.1, 48 x 32^3 (836 k) 181
+// and 157, 128^3 (1.06 M) 71.8 and 68.9, 4 x 128^3 467 and 432 us.
+static bool tt_wide(const ihg_ctx *c, int nr)
+{
+    return c->Ny <= TT_WIDE_MAX && c->M * nr < 300000;
 }
 
 // GW source pipeline on complex type C after the z pass: x pass, fused y
@@ -310,16 +363,42 @@ static int rhs_gw_t(ihg_ctx *c, C *Wk, const C *tw, const double *f,
         IHG_TRY(x_pass(c, Wk, -1, GW_NC, M, nr, rw));
     // y pass of the sources, TT projection and update_h: the sources
     // and h1, h2, dh1, dh2 in; the four h blocks of result out
+    const LineSet ls{(long)c->Nx * c->Mz, c->Mz, (long)c->Ny * c->Mz, c->Mz};
+    const double epb = !ep ? 0.0 : (ep->mode == RK4_FINAL ? 8.0 : 16.0);
+    const double bytes = (GW_NC * cs + (8.0 + epb) * 16.0) * M * nr;
+    if (tt_wide(c, nr))
+        return dispatch_len(c->Ny, [&](auto Lc) {
+            constexpr int L = decltype(Lc)::value;
+            if constexpr (L <= TT_WIDE_MAX) {
+                using TT = TTWide<L>;
+                const dim3 grid((unsigned)((ls.nlines + TT::B - 1) / TT::B), 1, nr);
+                return timed(c, F_TT_UPDATE_H, bytes, [&]() {
+                    if (ep)
+                        hipLaunchKernelGGL((k_y_tt_wide<L, C, true>), grid,
+                                           dim3(TT::WG), 0, c->stream, Wk, M, f,
+                                           result, N, c->Next, c->Ntot, c->kg,
+                                           c->dscal, ls, tw, e, rw,
+                                           gw_axis(c->kg), *ep);
+                    else
+                        hipLaunchKernelGGL((k_y_tt_wide<L, C, false>), grid,
+                                           dim3(TT::WG), 0, c->stream, Wk, M, f,
+                                           result, N, c->Next, c->Ntot, c->kg,
+                                           c->dscal, ls, tw, e, rw,
+                                           gw_axis(c->kg), Rk4Ep{});
+                    return hip_check(hipGetLastError(), "k_y_tt_wide");
+                });
+            } else {
+                return set_error("no wide TT pass for %d points", L);
+            }
+        });
     if constexpr (std::is_same<C, double2>::value) {
         if (ep)
             return dispatch_rk4_len(c->Ny, [&](auto Lc) {
                 constexpr int L = decltype(Lc)::value;
                 using TP = TTPlan<L>;
                 constexpr int B = TP::WG / (L / TP::P::E);
-                const LineSet ls{(long)c->Nx * c->Mz, c->Mz, (long)c->Ny * c->Mz, c->Mz};
                 const unsigned nb = (unsigned)((ls.nlines + B - 1) / B);
-                const double epb = ep->mode == RK4_FINAL ? 8.0 : 16.0;
-                return timed(c, F_TT_UPDATE_H, (GW_NC * 16.0 + (8.0 + epb) * 16.0) * M * nr, [&]() {
+                return timed(c, F_TT_UPDATE_H, bytes, [&]() {
                     hipLaunchKernelGGL((k_y_tt_update_h_rk4<L, TP::WG, typename TP::P>),
                                        dim3(nb, 1, nr), dim3(TP::WG), 0, c->stream, Wk,
                                        M, f, result, N, c->Next, c->Ntot, c->kg,
@@ -334,10 +413,8 @@ static int rhs_gw_t(ihg_ctx *c, C *Wk, const C *tw, const double *f,
         constexpr int L = decltype(Lc)::value;
         using TP = TTPlan<L>;
         constexpr int B = TP::WG / (L / TP::P::E);
-        // lines along y: one per (x, kz); points Mz apart
-        const LineSet ls{(long)c->Nx * c->Mz, c->Mz, (long)c->Ny * c->Mz, c->Mz};
         const unsigned nb = (unsigned)((ls.nlines + B - 1) / B);
-        return timed(c, F_TT_UPDATE_H, (GW_NC * cs + 8.0 * 16.0) * M * nr, [&]() {
+        return timed(c, F_TT_UPDATE_H, bytes, [&]() {
             hipLaunchKernelGGL((k_y_tt_update_h<L, TP::WG, typename TP::P, C>),
                                dim3(nb, 1, nr), dim3(TP::WG), 0, c->stream, Wk,
                                M, f, result, N, c->Next, c->Ntot, c->kg,

@@ -426,8 +426,28 @@ inline ZRhsArgs<C> z_rhs_args(const ihg_ctx *c, const double *f,
 }
 
 // rho_mean, pressure_mean (src/toolbox.c:241-242) and da (src/toolbox.c:87)
+// of realization r (one thread; EP: the RK4 epilogue of the scale factor)
+template <bool EP>
+__device__ __forceinline__ void means_store(unsigned r, double rm, double pm,
+                                            const double *__restrict__ f,
+                                            double *__restrict__ result,
+                                            long Ntot,
+                                            double *__restrict__ dscal,
+                                            const Ens &e, const Rk4Ep &ep)
+{
+    f += r * e.f;
+    result += r * e.f;
+    dscal += r * e.s;
+    dscal[S_RHO_MEAN] = rm;
+    dscal[S_P_MEAN] = pm;
+    const double da = f[Ntot - 1] * sqrt(rm / 3.0);
+    if constexpr (EP)
+        rk4_ep_one(ep.shifted(r * e.f), Ntot - 1, da, result + Ntot - 1);
+    else
+        result[Ntot - 1] = da;
+}
+
 // (one work-group per realization r; sh: MEANS_WG / 64 doubles of LDS)
-// EP: the RK4 epilogue of the scale factor's slope
 constexpr int MEANS_WG = 1024;
 template <bool EP = false>
 __device__ __forceinline__ void means_body(
@@ -437,9 +457,6 @@ __device__ __forceinline__ void means_body(
     const Rk4Ep &ep = Rk4Ep{})
 {
     partials += r * e.p;
-    f += r * e.f;
-    result += r * e.f;
-    dscal += r * e.s;
     // (rho, p) pairs as 16-byte loads, four in flight per thread
     const double2 *p2 = reinterpret_cast<const double2 *>(partials);
     double s0 = 0.0, s1 = 0.0;
@@ -451,35 +468,65 @@ __device__ __forceinline__ void means_body(
     }
     s0 = block_reduce<OpSum>(s0, sh, MEANS_WG);
     s1 = block_reduce<OpSum>(s1, sh, MEANS_WG);
-    if (threadIdx.x == 0) {
-        const double rm = s0 / N, pm = s1 / N;
-        dscal[S_RHO_MEAN] = rm;
-        dscal[S_P_MEAN] = pm;
-        const double da = f[Ntot - 1] * sqrt(rm / 3.0);
-        if constexpr (EP)
-            rk4_ep_one(ep.shifted(r * e.f), Ntot - 1, da, result + Ntot - 1);
-        else
-            result[Ntot - 1] = da;
+    if (threadIdx.x == 0)
+        means_store<EP>(r, s0 / N, s1 / N, f, result, Ntot, dscal, e, ep);
+}
+
+// The sums of means_body by a work-group of RED_WG threads, bit for bit: a
+// thread stands for MEANS_WG / RED_WG of its threads, and the wavefronts' sums
+// are added in its order.  sh: 2 MEANS_WG / 64 doubles; every thread gets the
+// sums; synchronises.
+__device__ __forceinline__ void means_sums(const double *__restrict__ partials,
+                                           int nparts, double *sh, double &s0,
+                                           double &s1)
+{
+    constexpr int V = MEANS_WG / RED_WG, NWV = MEANS_WG / 64;
+    const double2 *p2 = reinterpret_cast<const double2 *>(partials);
+    double a[V], b[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        a[v] = b[v] = 0.0;
+        for (int i = (int)threadIdx.x + RED_WG * v; i < nparts; i += MEANS_WG) {
+            const double2 q = p2[i];
+            a[v] += q.x;
+            b[v] += q.y;
+        }
+    }
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        a[v] = wave_reduce<OpSum>(a[v]);
+        b[v] = wave_reduce<OpSum>(b[v]);
+        if (lane == 0) {
+            sh[w + (RED_WG / 64) * v] = a[v];
+            sh[NWV + w + (RED_WG / 64) * v] = b[v];
+        }
+    }
+    __syncthreads();
+    s0 = sh[0];
+    s1 = sh[NWV];
+#pragma unroll
+    for (int i = 1; i < NWV; ++i) {
+        s0 += sh[i];
+        s1 += sh[NWV + i];
     }
 }
 
 // update_phi_psi (src/toolbox.c:282-299); the part A of the slope of dphi and
 // p were parked in result[0..N) and result[3N..4N) by k_z_rhs
 // (work-group bx of gx on realization z; EP: the RK4 epilogue of the four
-// blocks' slopes)
+// blocks' slopes; rm, pm: the means of rho and p)
 template <bool NT, bool EP = false>
 __device__ __forceinline__ void update_phi_psi_body(
     unsigned bx, unsigned gx, unsigned z, const double *__restrict__ f,
-    double *__restrict__ result, long N,
-    const double *__restrict__ dscal, const Ens &e, const Rk4Ep &ep0 = Rk4Ep{})
+    double *__restrict__ result, long N, double rm, double pm, const Ens &e,
+    const Rk4Ep &ep0 = Rk4Ep{})
 {
     f += z * e.f;
     result += z * e.f;
-    dscal += z * e.s;
     [[maybe_unused]] const Rk4Ep ep = EP ? ep0.shifted(z * e.f) : ep0;
-    const double hubble = sqrt(dscal[S_RHO_MEAN] / 3.0);
+    const double hubble = sqrt(rm / 3.0);
     const double h3 = 3.0 * hubble;
-    const double pm = dscal[S_P_MEAN];
     // pairs of points (16-byte loads and stores; N is even and every block
     // starts 16-byte aligned)
     const long stride = (long)gx * RED_WG;
@@ -509,13 +556,16 @@ __device__ __forceinline__ void update_phi_psi_body(
     }
 }
 
-template <bool NT>
-__global__ __launch_bounds__(RED_WG) void k_update_phi_psi(
-    const double *__restrict__ f, double *__restrict__ result, long N,
-    const double *__restrict__ dscal, Ens e)
+// the means of realization z from k_means
+template <bool NT, bool EP = false>
+__device__ __forceinline__ void update_after_means_body(
+    unsigned bx, unsigned gx, unsigned z, const double *__restrict__ f,
+    double *__restrict__ result, long N, const double *__restrict__ dscal,
+    const Ens &e, const Rk4Ep &ep = Rk4Ep{})
 {
-    update_phi_psi_body<NT>(blockIdx.x, gridDim.x, blockIdx.z, f, result, N,
-                            dscal, e);
+    const double *d = dscal + z * e.s;
+    update_phi_psi_body<NT, EP>(bx, gx, z, f, result, N, d[S_RHO_MEAN],
+                                d[S_P_MEAN], e, ep);
 }
 
 // ---------------------------------------------------------------------------
@@ -659,6 +709,49 @@ __host__ __device__ constexpr int tt_lds()
     return 2 * (WG / (L / P::E)) * Lds<L>::PITCH + L;
 }
 
+// update_h at one point (src/toolbox.c:311-346) from the two projected sources
+struct HUpdate {
+    double a2, h3, pm;
+    double2 *r2;
+    long Nh1, Nh2, Ndh1, Ndh2; // offsets of the h blocks in complex values
+    __device__ __forceinline__ HUpdate(const double *f, double *result, long N,
+                                       long Next, long Ntot, const double *dscal)
+    {
+        const double aa = f[Ntot - 1];
+        a2 = aa * aa;
+        h3 = 3.0 * sqrt(dscal[S_RHO_MEAN] / 3.0);
+        pm = dscal[S_P_MEAN];
+        r2 = reinterpret_cast<double2 *>(result);
+        Nh1 = 2 * N;
+        Nh2 = Nh1 + Next / 2;
+        Ndh1 = Nh2 + Next / 2;
+        Ndh2 = Ndh1 + Next / 2;
+    }
+    template <bool EP>
+    __device__ __forceinline__ void point(long i, double ksq, double2 h1,
+                                          double2 h2, double2 d1, double2 d2,
+                                          double2 s0, double2 s1,
+                                          const Rk4Ep &ep) const
+    {
+        const double tmp = -(2.0 * pm + ksq / a2);
+        const double2 v1 = make_double2(tmp * h1.x - h3 * d1.x + 2.0 * s0.x / a2,
+                                        tmp * h1.y - h3 * d1.y + 2.0 * s0.y / a2);
+        const double2 v2 = make_double2(tmp * h2.x - h3 * d2.x + 2.0 * s1.x / a2,
+                                        tmp * h2.y - h3 * d2.y + 2.0 * s1.y / a2);
+        if constexpr (EP) {
+            rk4_ep_pair<false>(ep, Nh1 + i, d1, r2 + Nh1 + i);
+            rk4_ep_pair<false>(ep, Nh2 + i, d2, r2 + Nh2 + i);
+            rk4_ep_pair<false>(ep, Ndh1 + i, v1, r2 + Ndh1 + i);
+            rk4_ep_pair<false>(ep, Ndh2 + i, v2, r2 + Ndh2 + i);
+        } else {
+            r2[Nh1 + i] = d1;
+            r2[Nh2 + i] = d2;
+            r2[Ndh1 + i] = v1;
+            r2[Ndh2 + i] = v2;
+        }
+    }
+};
+
 // Last pass of the GW sources: y transforms of the components (z and x
 // passes done), the TT projection, and update_h (src/toolbox.c:311-346):
 //   dh = hdot,  dhdot = -(2 p_mean + k^2/a^2) h - 3 H hdot + 2 S^TT / a^2
@@ -787,38 +880,14 @@ __device__ __forceinline__ void y_tt_update_h_body(
     if constexpr (!EARLY) load_h();
     if (!act)
         return;
-    const double aa = f[Ntot - 1];
-    const double a2 = aa * aa;
-    const double hubble = sqrt(dscal[S_RHO_MEAN] / 3.0);
-    const double h3 = 3.0 * hubble;
-    const double pm = dscal[S_P_MEAN];
-    double2 *r2 = reinterpret_cast<double2 *>(result);
+    const HUpdate hu(f, result, N, Next, Ntot, dscal);
+    const Rk4Ep ep = EP ? ep0.shifted(bk.z * e.f) : ep0;
 #pragma unroll
     for (int s = 0; s < E; ++s) {
         const int n = last_point<L, P>(j, s);
-        const long i = base + n * st;
-        const double ksq = kg.ksq(ix, n, iz);
-        const double2 h1 = h1v[s], h2 = h2v[s], d1 = d1v[s], d2 = d2v[s];
-        if constexpr (!EP) {
-            r2[Nh1 / 2 + i] = d1;
-            r2[Nh2 / 2 + i] = d2;
-        }
-        const double tmp = -(2.0 * pm + ksq / a2);
-        const double s0x = o0[s].x, s0y = o0[s].y, s1x = o1[s].x, s1y = o1[s].y;
-        const double2 v1 = make_double2(tmp * h1.x - h3 * d1.x + 2.0 * s0x / a2,
-                                        tmp * h1.y - h3 * d1.y + 2.0 * s0y / a2);
-        const double2 v2 = make_double2(tmp * h2.x - h3 * d2.x + 2.0 * s1x / a2,
-                                        tmp * h2.y - h3 * d2.y + 2.0 * s1y / a2);
-        if constexpr (EP) {
-            const Rk4Ep ep = ep0.shifted(bk.z * e.f);
-            rk4_ep_pair<false>(ep, Nh1 / 2 + i, d1, r2 + Nh1 / 2 + i);
-            rk4_ep_pair<false>(ep, Nh2 / 2 + i, d2, r2 + Nh2 / 2 + i);
-            rk4_ep_pair<false>(ep, Ndh1 / 2 + i, v1, r2 + Ndh1 / 2 + i);
-            rk4_ep_pair<false>(ep, Ndh2 / 2 + i, v2, r2 + Ndh2 / 2 + i);
-        } else {
-            r2[Ndh1 / 2 + i] = v1;
-            r2[Ndh2 / 2 + i] = v2;
-        }
+        hu.template point<EP>(base + n * st, kg.ksq(ix, n, iz), h1v[s], h2v[s],
+                              d1v[s], d2v[s], make_double2(o0[s].x, o0[s].y),
+                              make_double2(o1[s].x, o1[s].y), ep);
     }
 }
 
@@ -834,5 +903,129 @@ __global__ __launch_bounds__(WG) void k_y_tt_update_h(
                                     Ntot, kg, dscal, ls, tw, e, rw, ga);
 }
 
+
+// ---------------------------------------------------------------------------
+// The same pass for grids that leave the chip idle: latency bounds it (one 64^3
+// grid is 528 wavefronts, each running five transforms in turn), so the five
+// components of a tile are transformed at the same time by a fifth of the
+// work-group each, in one layout with work-group barriers, and after the last
+// stage every thread takes points of the tile: five spectra from LDS, the
+// projection in the order of tt_component, and update_h, whose inputs were
+// loaded before the transforms.  Line plans have the radices of TTPlan and the
+// sums their order, so the values are the same bit for bit.  7 x 16^3 with the
+// RK4 epilogue 13.3 -> 6.2 us, 3 x 32^3 16.3 -> 7.4, 64^3 13.1 -> 12.0; the
+// rule of tt_wide has the sizes where it loses.
+// ---------------------------------------------------------------------------
+template <int L> struct TTWidePlan { using P = typename TTPlan<L>::P; static constexpr int B = 8; };
+template <> struct TTWidePlan<4> { using P = PlanT<4, 2, 2>; static constexpr int B = 64; };
+template <> struct TTWidePlan<8> { using P = PlanT<4, 4, 2>; static constexpr int B = 32; };
+template <> struct TTWidePlan<16> { using P = PlanT<4, 4, 4>; static constexpr int B = 16; };
+template <> struct TTWidePlan<128> { using P = PlanT<8, 4, 4, 4, 2>; static constexpr int B = 8; };
+
+// lines up to 128 points: 256 would need 175 KB of LDS for 128-byte runs
+constexpr int TT_WIDE_MAX = 128;
+
+template <int L>
+struct TTWide {
+    using P = typename TTWidePlan<L>::P;
+    static constexpr int B = TTWidePlan<L>::B, T = L / P::E;
+    static constexpr int WG = GW_NC * B * T, LDS = GW_NC * B * Lds<L>::PITCH;
+    static_assert(WG % 64 == 0 && WG <= 1024, "whole wavefronts");
+};
+
+template <int L, class C, bool EP>
+__device__ __forceinline__ void y_tt_wide_body(
+    const Blk &bk, C *lds, const C *W, long M, const double *__restrict__ f,
+    double *__restrict__ result, long N, long Next, long Ntot,
+    const KGeom &kg, const double *__restrict__ dscal, const LineSet &ls,
+    const C *__restrict__ tw, const Ens &e, long rw, GwAxis ga,
+    const Rk4Ep &ep0)
+{
+    using TT = TTWide<L>;
+    using P = typename TT::P;
+    using R = typename CT<C>::R;
+    constexpr int B = TT::B, T = TT::T, WG = TT::WG, PITCH = Lds<L>::PITCH;
+    constexpr int NP = (B * L + WG - 1) / WG; // points per thread
+    W += bk.z * rw;
+    f += bk.z * e.f;
+    result += bk.z * e.f;
+    dscal += bk.z * e.s;
+    const int tid = threadIdx.x;
+    const long line0 = (long)tile_x<true>(bk) * B;
+    const long st = ls.stride;
+    // the transform of component c: thread j of line b; idle lines transform
+    // line 0 (in bounds)
+    const int c = tid / (B * T), t = tid % (B * T), b = t % B, j = t / B;
+    const long line = line0 + b;
+    const C *src = W + c * M + ls.base(line < ls.nlines ? line : 0);
+    C buf[P::E];
+#pragma unroll
+    for (int s = 0; s < P::E; ++s)
+        buf[s] = src[(long)stage1_point<L, P>(j, s) * st];
+    // this thread's points: line pb, point pn; h and hdot ahead
+    const HUpdate hu(f, result, N, Next, Ntot, dscal);
+    const double2 *f2 = reinterpret_cast<const double2 *>(f);
+    double2 h1[NP], h2[NP], d1[NP], d2[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const int q = tid + p * WG, pb = q % B, pn = q / B;
+        const long pl = line0 + pb;
+        const long i = pn < L && pl < ls.nlines ? ls.base(pl) + pn * st : 0;
+        h1[p] = f2[hu.Nh1 + i];
+        h2[p] = f2[hu.Nh2 + i];
+        d1[p] = f2[hu.Ndh1 + i];
+        d2[p] = f2[hu.Ndh2 + i];
+    }
+    fft_line<L, -1, true, false, P>(lds + (c * B + b) * PITCH, j, tw,
+                                    [&](int s, int) { return buf[s]; });
+    const Rk4Ep ep = EP ? ep0.shifted(bk.z * e.f) : ep0;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const int q = tid + p * WG, pb = q % B, pn = q / B;
+        const long pl = line0 + pb;
+        if (pn >= L || pl >= ls.nlines) continue;
+        const int ix = (int)(pl / kg.Mz), iz = (int)(pl - (long)ix * kg.Mz);
+        const bool zero = ix == 0 && iz == 0 && pn == 0;
+        const bool b1 = fabs(kg.kzf(iz)) > DBL_EPSILON;
+        const double ksq = kg.ksq(ix, pn, iz);
+        const R inv = zero ? (R)0 : (R)(1.0 / ksq);
+        const R kx = (R)kg.kxf(ix), ky = (R)kg.kyf(pn), kz = (R)kg.kzf(iz);
+        const C *v = lds + pb * PITCH + Lds<L>::idx(pn);
+        C o0, o1;
+        auto add = [&](auto kc) {
+            constexpr int K = decltype(kc)::value;
+            R al, be;
+            tt_source_coef<K>(kx, ky, kz, inv, b1, zero, ga.m, al, be);
+            const C u = v[K * B * PITCH];
+            if constexpr (K == 0) {
+                o0 = CT<C>::make(al * u.x, al * u.y);
+                o1 = CT<C>::make(be * u.x, be * u.y);
+            } else {
+                o0 = CT<C>::make(o0.x + al * u.x, o0.y + al * u.y);
+                o1 = CT<C>::make(o1.x + be * u.x, o1.y + be * u.y);
+            }
+        };
+        add(std::integral_constant<int, 0>{});
+        add(std::integral_constant<int, 1>{});
+        add(std::integral_constant<int, 2>{});
+        add(std::integral_constant<int, 3>{});
+        add(std::integral_constant<int, 4>{});
+        hu.template point<EP>(ls.base(pl) + pn * st, ksq, h1[p], h2[p], d1[p],
+                              d2[p], make_double2(o0.x, o0.y),
+                              make_double2(o1.x, o1.y), ep);
+    }
+}
+
+template <int L, class C, bool EP>
+__global__ __launch_bounds__(TTWide<L>::WG) void k_y_tt_wide(
+    const C *W, long M, const double *__restrict__ f,
+    double *__restrict__ result, long N, long Next, long Ntot, KGeom kg,
+    const double *__restrict__ dscal, LineSet ls, const C *__restrict__ tw,
+    Ens e, long rw, GwAxis ga, Rk4Ep ep)
+{
+    __shared__ C lds[TTWide<L>::LDS];
+    y_tt_wide_body<L, C, EP>(hw_blk(), lds, W, M, f, result, N, Next, Ntot, kg,
+                             dscal, ls, tw, e, rw, ga, ep);
+}
 
 } // namespace ihg
