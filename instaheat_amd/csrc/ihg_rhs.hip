@@ -75,7 +75,7 @@ __global__ __launch_bounds__(RED_WG) void k_update_phi_psi_rk4(
 // k_means and the update in one launch for few partial sums: every
 // work-group adds them up itself (the same sums bit for bit), the first of a
 // realization also stores the means and does the scale factor.
-template <bool EP>
+template <bool EP, bool AHEAD>
 __global__ __launch_bounds__(RED_WG) void k_means_update(
     const double *__restrict__ partials, int nparts, long N,
     const double *__restrict__ f, double *__restrict__ result, long Ntot,
@@ -88,8 +88,8 @@ __global__ __launch_bounds__(RED_WG) void k_means_update(
     const double rm = s0 / N, pm = s1 / N;
     if (blockIdx.x == 0 && threadIdx.x == 0)
         means_store<EP>(z, rm, pm, f, result, Ntot, dscal, e, ep);
-    update_phi_psi_body<false, EP>(blockIdx.x, gridDim.x, z, f, result, N, rm,
-                                   pm, e, ep);
+    update_phi_psi_body<false, EP, AHEAD>(blockIdx.x, gridDim.x, z, f, result, N,
+                                          rm, pm, e, ep);
 }
 
 template <int L, int WG, class P>
@@ -293,18 +293,24 @@ int rhs_core(ihg_ctx *c, double *f, double *result, int output, int filtered,
     // the epilogue reads y (and k1..k3) and writes the stage output beside
     // the slope: 2 (stage) or 4 (final, no slope written) more blocks
     const double ep_blocks = !ep ? 0.0 : (ep->mode == RK4_FINAL ? 4.0 : 8.0);
-    const dim3 ugrid(nblocks(N, RED_WG * 4, 65536), 1, nr);
+    // one pair of points a thread on small grids (32^3 with the epilogue 5.1
+    // against 5.9 us, 7 x 16^3 + 3 x 32^3 5.9 and 6.8), two on larger ones
+    // (64^3 6.2 against 7.0 us: the work-groups' sums count)
+    const bool small = N * nr < 200000;
+    const dim3 ugrid(nblocks(N, small ? RED_WG * 2 : RED_WG * 4, 65536), 1, nr);
     // One launch where the partial sums are few (64^3 has 512): 4.6 us against
     // 3.6 + 3.0 at 16^3, 6.3 against 4.4 + 5.2 at 64^3; every work-group then
     // reads all of them (at most 16 KB, from L2).
     if (nparts <= MEANS_WG && 4.0 * 8.0 * (double)N * nr < NT_BYTES)
         return timed(c, F_UPDATE, (9.0 + ep_blocks) * 8.0 * N * nr, [&]() {
             if (ep)
-                hipLaunchKernelGGL(k_means_update<true>, ugrid, dim3(RED_WG), 0,
+                hipLaunchKernelGGL((small ? k_means_update<true, true>
+                                          : k_means_update<true, false>),
+                                   ugrid, dim3(RED_WG), 0,
                                    c->stream, c->partials, nparts, N, f, result,
                                    c->Ntot, c->dscal, e, *ep);
             else
-                hipLaunchKernelGGL(k_means_update<false>, ugrid, dim3(RED_WG), 0,
+                hipLaunchKernelGGL((k_means_update<false, false>), ugrid, dim3(RED_WG), 0,
                                    c->stream, c->partials, nparts, N, f, result,
                                    c->Ntot, c->dscal, e, Rk4Ep{});
             return hip_check(hipGetLastError(), "k_means_update");

@@ -515,8 +515,9 @@ __device__ __forceinline__ void means_sums(const double *__restrict__ partials,
 // update_phi_psi (src/toolbox.c:282-299); the part A of the slope of dphi and
 // p were parked in result[0..N) and result[3N..4N) by k_z_rhs
 // (work-group bx of gx on realization z; EP: the RK4 epilogue of the four
-// blocks' slopes; rm, pm: the means of rho and p)
-template <bool NT, bool EP = false>
+// blocks' slopes, AHEAD with its loads before the first store; rm, pm: the
+// means of rho and p)
+template <bool NT, bool EP = false, bool AHEAD = false>
 __device__ __forceinline__ void update_phi_psi_body(
     unsigned bx, unsigned gx, unsigned z, const double *__restrict__ f,
     double *__restrict__ result, long N, double rm, double pm, const Ens &e,
@@ -537,16 +538,27 @@ __device__ __forceinline__ void update_phi_psi_body(
         const double2 dph = ld2<NT>(F + H + i), ps = ld2<NT>(F + 2 * H + i),
                       dps = ld2<NT>(F + 3 * H + i);
         const double2 A = ld2<NT>(Rs + i), pr = ld2<NT>(Rs + 3 * H + i);
+        [[maybe_unused]] Rk4In in[4];
+        if constexpr (EP && AHEAD) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) in[q] = rk4_ep_load<NT>(ep, q * H + i);
+        }
         const double2 r1 = make_double2(A.x - (h3 - 4.0 * dps.x) * dph.x,
                                         A.y - (h3 - 4.0 * dps.y) * dph.y);
         const double2 r3 = make_double2(
             0.5 * pr.x + (ps.x - 0.5) * pm - 4.0 * hubble * dps.x,
             0.5 * pr.y + (ps.y - 0.5) * pm - 4.0 * hubble * dps.y);
         if constexpr (EP) {
-            rk4_ep_pair<NT>(ep, i, dph, Rs + i);
-            rk4_ep_pair<NT>(ep, H + i, r1, Rs + H + i);
-            rk4_ep_pair<NT>(ep, 2 * H + i, dps, Rs + 2 * H + i);
-            rk4_ep_pair<NT>(ep, 3 * H + i, r3, Rs + 3 * H + i);
+            auto put = [&](int q, double2 k) {
+                if constexpr (AHEAD)
+                    rk4_ep_store<NT>(ep, q * H + i, in[q], k, Rs + q * H + i);
+                else
+                    rk4_ep_pair<NT>(ep, q * H + i, k, Rs + q * H + i);
+            };
+            put(0, dph);
+            put(1, r1);
+            put(2, dps);
+            put(3, r3);
         } else {
             st2<NT>(Rs + i, dph);
             st2<NT>(Rs + H + i, r1);
@@ -727,7 +739,8 @@ struct HUpdate {
         Ndh1 = Nh2 + Next / 2;
         Ndh2 = Ndh1 + Next / 2;
     }
-    template <bool EP>
+    // AHEAD: what the epilogue reads of the four blocks is loaded first
+    template <bool EP, bool AHEAD>
     __device__ __forceinline__ void point(long i, double ksq, double2 h1,
                                           double2 h2, double2 d1, double2 d2,
                                           double2 s0, double2 s1,
@@ -739,10 +752,23 @@ struct HUpdate {
         const double2 v2 = make_double2(tmp * h2.x - h3 * d2.x + 2.0 * s1.x / a2,
                                         tmp * h2.y - h3 * d2.y + 2.0 * s1.y / a2);
         if constexpr (EP) {
-            rk4_ep_pair<false>(ep, Nh1 + i, d1, r2 + Nh1 + i);
-            rk4_ep_pair<false>(ep, Nh2 + i, d2, r2 + Nh2 + i);
-            rk4_ep_pair<false>(ep, Ndh1 + i, v1, r2 + Ndh1 + i);
-            rk4_ep_pair<false>(ep, Ndh2 + i, v2, r2 + Ndh2 + i);
+            [[maybe_unused]] Rk4In in[4];
+            if constexpr (AHEAD) {
+                in[0] = rk4_ep_load<false>(ep, Nh1 + i);
+                in[1] = rk4_ep_load<false>(ep, Nh2 + i);
+                in[2] = rk4_ep_load<false>(ep, Ndh1 + i);
+                in[3] = rk4_ep_load<false>(ep, Ndh2 + i);
+            }
+            auto put = [&](int q, long at, double2 k) {
+                if constexpr (AHEAD)
+                    rk4_ep_store<false>(ep, at, in[q], k, r2 + at);
+                else
+                    rk4_ep_pair<false>(ep, at, k, r2 + at);
+            };
+            put(0, Nh1 + i, d1);
+            put(1, Nh2 + i, d2);
+            put(2, Ndh1 + i, v1);
+            put(3, Ndh2 + i, v2);
         } else {
             r2[Nh1 + i] = d1;
             r2[Nh2 + i] = d2;
@@ -885,7 +911,7 @@ __device__ __forceinline__ void y_tt_update_h_body(
 #pragma unroll
     for (int s = 0; s < E; ++s) {
         const int n = last_point<L, P>(j, s);
-        hu.template point<EP>(base + n * st, kg.ksq(ix, n, iz), h1v[s], h2v[s],
+        hu.template point<EP, false>(base + n * st, kg.ksq(ix, n, iz), h1v[s], h2v[s],
                               d1v[s], d2v[s], make_double2(o0[s].x, o0[s].y),
                               make_double2(o1[s].x, o1[s].y), ep);
     }
@@ -1010,7 +1036,7 @@ __device__ __forceinline__ void y_tt_wide_body(
         add(std::integral_constant<int, 2>{});
         add(std::integral_constant<int, 3>{});
         add(std::integral_constant<int, 4>{});
-        hu.template point<EP>(ls.base(pl) + pn * st, ksq, h1[p], h2[p], d1[p],
+        hu.template point<EP, true>(ls.base(pl) + pn * st, ksq, h1[p], h2[p], d1[p],
                               d2[p], make_double2(o0.x, o0.y),
                               make_double2(o1.x, o1.y), ep);
     }

@@ -139,6 +139,46 @@ __device__ __forceinline__ void rk4_ep_pair(const Rk4Ep &ep, long p, double2 k,
     }
 }
 
+// The same in two parts: what the epilogue reads of the pair, and the stores
+// once its slope k is known.  On small grids a kernel loads the pairs of all
+// its blocks before the first store: a load behind a store that may alias it
+// waits (the update of one 32^3 grid 7.9 -> 5.1 us).  Larger ones have
+// wavefronts enough and keep their registers (4 x 128^3: 262 us, with the
+// loads ahead 285).
+struct Rk4In {
+    double2 y, a, b, c;
+};
+template <bool NT>
+__device__ __forceinline__ Rk4In rk4_ep_load(const Rk4Ep &ep, long p)
+{
+    Rk4In v;
+    if (ep.mode == RK4_FINAL) {
+        v.y = ld2<NT>(reinterpret_cast<const double2 *>(ep.out) + p);
+        v.a = ld2<NT>(reinterpret_cast<const double2 *>(ep.k1) + p);
+        v.b = ld2<NT>(reinterpret_cast<const double2 *>(ep.k2) + p);
+        v.c = ld2<NT>(reinterpret_cast<const double2 *>(ep.k3) + p);
+    } else {
+        v.y = ld2<NT>(reinterpret_cast<const double2 *>(ep.y) + p);
+    }
+    return v;
+}
+template <bool NT>
+__device__ __forceinline__ void rk4_ep_store(const Rk4Ep &ep, long p,
+                                             const Rk4In &v, double2 k,
+                                             double2 *kdst)
+{
+    k = make_double2(opaque(k.x), opaque(k.y));
+    double2 *o = reinterpret_cast<double2 *>(ep.out) + p; // FINAL: y, in place
+    if (ep.mode == RK4_FINAL) {
+        st2<NT>(o, make_double2(rk4_final_val(v.y.x, v.a.x, v.b.x, v.c.x, k.x, ep.dt),
+                                rk4_final_val(v.y.y, v.a.y, v.b.y, v.c.y, k.y, ep.dt)));
+    } else {
+        st2<NT>(kdst, k);
+        st2<NT>(o, make_double2(rk4_stage_val(v.y.x, k.x, ep.dt, ep.half),
+                                rk4_stage_val(v.y.y, k.y, ep.dt, ep.half)));
+    }
+}
+
 // one element i whose slope is k
 __device__ __forceinline__ void rk4_ep_one(const Rk4Ep &ep, long i, double k,
                                            double *kdst)
