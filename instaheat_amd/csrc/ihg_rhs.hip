@@ -231,6 +231,9 @@ static int deriv_pass(ihg_ctx *c, int len, const DerivXY &d, int naxes, int nr)
     });
 }
 
+// CUs of the chip: a work-group of the z pass with helper wavefronts fills one
+constexpr unsigned NUM_CU = 256;
+
 template <class C>
 static int z_pass(ihg_ctx *c, const double *f, double *result, int output,
                   const DerivIO &io, int nr, int &nparts)
@@ -258,8 +261,23 @@ static int z_pass(ihg_ctx *c, const double *f, double *result, int output,
         return timed(c, F_Z_RHS, bytes, [&]() {
             auto go = [&](auto gwc) {
                 constexpr bool G = decltype(gwc)::value;
-                if (wg == 64)
-                    hipLaunchKernelGGL((k_z_rhs<L, G, C, 64>), grid, dim3(64), 0, c->stream, a);
+                auto small = [&](auto wgc) {
+                    constexpr int WG = decltype(wgc)::value;
+                    hipLaunchKernelGGL((k_z_rhs<L, G, C, WG, (WG > 64)>), grid,
+                                       dim3(WG), 0, c->stream, a);
+                };
+                // Helper wavefronts while the work-groups, two wavefronts a
+                // SIMD at their registers, run all at once: five up to a
+                // work-group a CU (7 x 16^3 11.0 -> 7.7 us, 3 x 32^3 13.5 ->
+                // 9.8), three up to two (64^3, 512 work-groups: 15.4 -> 12.6;
+                // with five 15.7), none beyond (64 x 256 x 32, 1024: 18 us,
+                // with five 28).
+                if (wg == 64 && G && grid.x * nr <= NUM_CU)
+                    small(std::integral_constant<int, G ? 64 * GW_NC : 64>{});
+                else if (wg == 64 && G && grid.x * nr <= 2 * NUM_CU)
+                    small(std::integral_constant<int, G ? 192 : 64>{});
+                else if (wg == 64)
+                    small(std::integral_constant<int, 64>{});
                 else
                     hipLaunchKernelGGL((k_z_rhs<L, G, C, 256>), grid, dim3(256), 0, c->stream, a);
             };

@@ -121,16 +121,17 @@ template <int L> struct ZRhsTile {
     static constexpr int E = P::E, T = L / E, PITCH = Lds<L>::PITCH, LPW = 64 / T;
 };
 
-// LDS of the z pass in complex values: the lines, then the stage twiddles
+// LDS of the z pass in complex values: the lines, the stage twiddles, and with
+// helper wavefronts the three gradients of their 64 E points
 template <int L, int WG>
 __host__ __device__ constexpr int z_rhs_lines()
 {
     return WG / ZRhsTile<L>::T * ZRhsTile<L>::PITCH;
 }
-template <int L, int WG>
+template <int L, int WG, bool HELP = false>
 __host__ __device__ constexpr int z_rhs_lds()
 {
-    return z_rhs_lines<L, WG>() + L;
+    return z_rhs_lines<L, WG>() + L + (HELP ? 3 * 64 * ZRhsTile<L>::E : 0);
 }
 
 // work-groups of the z pass, and its partial sums (one pair a wavefront)
@@ -182,30 +183,42 @@ __device__ __forceinline__ R gw_source(R gx, R gy, R gz, int m)
     }
 }
 
-template <int L, bool GW, class C, int WG>
+// HELP: all wavefronts of the work-group serve the lines of one; the first does
+// the derivatives and the points, then shares the gradients through LDS, and
+// the source components are transformed side by side.  On a grid of fewer
+// wavefronts than the chip has SIMDs the chain of eight transforms bounds the
+// pass (the rule and its figures are at the launch).
+template <int L, bool GW, class C, int WG, bool HELP = false>
 __device__ __forceinline__ void z_rhs_body(const Blk &bk, double2 *lds,
                                            const ZRhsArgs<C> &a)
 {
+    static_assert(GW || !HELP, "the sources are what is shared");
     using TL = ZRhsTile<L>;
     using P = typename TL::P;
     using R = typename CT<C>::R;
     constexpr int E = TL::E, T = TL::T, PITCH = TL::PITCH, LPW = TL::LPW;
-    constexpr int NW = WG / 64, MZ = L / 2 + 1;
+    constexpr int NW = HELP ? 1 : WG / 64, MZ = L / 2 + 1;
     // The other inputs of a point are loaded ahead of the transforms where
     // too few wavefronts are there to hide their latency (single-wavefront
     // work-groups: 5.1 against 6.0 us at 32^3; the 64- and 128-point lines of
     // the GW pass: 137 against 151 us for 16 x 64^3, 278 against 293 for 4 x
     // 128^3), and at the point elsewhere (256^3 411 against 425 us, 128^3
     // without GW 24 against 28 us): the registers cost a wave a SIMD.
-    constexpr bool PRE = WG == 64 || (GW && (L == 64 || L == 128));
-    const int w = (int)threadIdx.x / 64, lane = (int)threadIdx.x % 64;
+    constexpr bool PRE = HELP || WG == 64 || (GW && (L == 64 || L == 128));
+    const int wv = (int)threadIdx.x / 64, lane = (int)threadIdx.x % 64;
+    const int w = HELP ? 0 : wv;
+    [[maybe_unused]] const int role = __builtin_amdgcn_readfirstlane(wv);
     const int j = lane % T;
     const long wave = (long)bk.x * NW + w, line0 = wave * LPW;
     const long line = line0 + lane / T;
     const bool act = line < a.nrows / 2; // idle lanes work on line 0
     const long ia = (act ? 2 * line : 0) * L; // row A; row B is L further
-    double2 *wl = lds + w * LPW * PITCH, *my = wl + lane / T * PITCH;
-    const double2 *tw = twiddles_to_lds_wave<L>(lds + z_rhs_lines<L, WG>(), a.tw);
+    double2 *wl = lds + wv * LPW * PITCH, *my = wl + lane / T * PITCH;
+    double2 *const ltw = lds + z_rhs_lines<L, WG>();
+    [[maybe_unused]] C gx[E], gy[E], gz[E];
+    const double2 *const tw = ltw - L;
+    if (!HELP || role == 0) {
+    twiddles_to_lds_wave<L>(ltw, a.tw);
     const double *__restrict__ f = a.f + bk.z * a.e.f;
     const double *__restrict__ lx = a.result + bk.z * a.e.f + a.N;
     const double *__restrict__ ly = lx + a.N;
@@ -271,7 +284,6 @@ __device__ __forceinline__ void z_rhs_body(const Blk &bk, double2 *lds,
     const double aa = f[a.Ntot - 1];
     const double a2 = aa * aa;
     double srho = 0.0, sp = 0.0;
-    [[maybe_unused]] C gx[E], gy[E], gz[E];
 #pragma unroll
     for (int s = 0; s < E; ++s) {
         const long i = ia + last_point<L, P>(j, s);
@@ -326,6 +338,27 @@ __device__ __forceinline__ void z_rhs_body(const Blk &bk, double2 *lds,
         part[0] = srho;
         part[1] = sp;
     }
+    }
+    if constexpr (HELP) {
+        C *const g = reinterpret_cast<C *>(ltw + L) + lane;
+        if (role == 0) {
+#pragma unroll
+            for (int s = 0; s < E; ++s) {
+                g[64 * s] = gx[s];
+                g[64 * (E + s)] = gy[s];
+                g[64 * (2 * E + s)] = gz[s];
+            }
+        }
+        lds_barrier();
+        if (role != 0) {
+#pragma unroll
+            for (int s = 0; s < E; ++s) {
+                gx[s] = g[64 * s];
+                gy[s] = g[64 * (E + s)];
+                gz[s] = g[64 * (2 * E + s)];
+            }
+        }
+    }
     if constexpr (GW) {
         C *const cl = reinterpret_cast<C *>(wl); // the wavefront's own lines
         C *const cmy = cl + lane / T * PITCH;
@@ -339,6 +372,7 @@ __device__ __forceinline__ void z_rhs_body(const Blk &bk, double2 *lds,
             twc = a.twc;
         auto comp = [&](auto kc) {
             constexpr int K = decltype(kc)::value;
+            if (HELP && role != K % (WG / 64)) return;
             line_sync<true>(); // earlier LDS reads of these lines are done
             fft_line_impl<L, -1, true, false, P, C, true>(
                 cmy, cmy, j, twc,
@@ -362,11 +396,11 @@ __device__ __forceinline__ void z_rhs_body(const Blk &bk, double2 *lds,
     }
 }
 
-template <int L, bool GW, class C, int WG>
+template <int L, bool GW, class C, int WG, bool HELP = false>
 __global__ __launch_bounds__(WG) void k_z_rhs(ZRhsArgs<C> a)
 {
-    __shared__ double2 lds[z_rhs_lds<L, WG>()];
-    z_rhs_body<L, GW, C, WG>(hw_blk(), lds, a);
+    __shared__ double2 lds[z_rhs_lds<L, WG, HELP>()];
+    z_rhs_body<L, GW, C, WG, HELP>(hw_blk(), lds, a);
 }
 
 // The derivative passes of nr realizations of a context: the field they
