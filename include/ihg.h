@@ -249,7 +249,8 @@ int ihg_mk_rhs_ensemble(ihg_ctx *c, double t, double *f, double *result,
  *   IHG_RK4_STAGE: out = y + dt k / 2 (half = 1) or y + dt k (half = 0),
  *                  the next stage's input (out differs from f, result, y);
  *   IHG_RK4_FINAL: y = y + dt (k1 + 2 k2 + 2 k3 + k) / 6 in place (y differs
- *                  from f and result); the slope k itself is not stored.
+ *                  from f and result); the slope k itself is not stored, and
+ *                  result is left with intermediate values.
  * The values equal ihg_mk_rhs_ensemble followed by ihg_rk4_stage /
  * ihg_rk4_final bit for bit, with one sweep of the state fewer per stage
  * (on contexts without the fused kernels -- the FP32 GW source, or GW
@@ -274,10 +275,12 @@ int ihg_mk_rhs_rk4(ihg_ctx *c, double t, double *f, double *result,
  * single) contexts of cubic grids of 16, 32, 64 or 128 points, FP64.
  * ihg_group_mk_rhs does what ihg_mk_rhs_ensemble does on every context, and
  * ihg_group_rk4_stage / ihg_group_rk4_final what ihg_rk4_stage /
- * ihg_rk4_final do, but each pass of all contexts is ONE launch: its work-
- * groups come from a table of segments, one per context, each running the
- * per-context kernel's body on its own grid, so the values are those of the
- * per-context calls bit for bit.  Array arguments hold one pointer per
+ * ihg_rk4_final do, but each pass of all contexts is ONE launch (the
+ * derivative and z passes one for the contexts with GW and one for those
+ * without, the filter's x pass one for lines of up to 64 points and one for
+ * 128): its work-groups come from a table of segments, one per context, each
+ * running the per-context kernel's body on its own grid, so the values are
+ * those of the per-context calls bit for bit.  Array arguments hold one pointer per
  * context, in the order of ihg_group_create.  Launches go to the FIRST
  * context's stream (capture them with ihg_graph_begin on that context); the
  * other contexts' streams must be idle (ihg_sync) before grouped calls and
