@@ -78,7 +78,14 @@ struct FilterFac {
 // of the smallest Nyquist wave number, so that a difference is not rounded at
 // the size of a much larger product: with m = z on a box resolved more finely
 // along z the slopes of h lost a factor of 2.5 (FP32, 4 x 4 x 512 points on a
-// cube).
+// cube).  Error of the projected source with FP32 products against six
+// components of products of rounded gradients, over white, k^-1 .. k^-3 and
+// plane-wave fields, both polarizations (geometric mean per box): 0.87 at 16^3,
+// 0.91 at 64^3 and 128^3, 0.94 for spacings of 1 : 2 : 0.5; random fields 0.9 to
+// 1.0 on cubes.  The least favourable is a plane wave along m, whose rounding
+// enters two components: 1.25 at 64^3 (the other polarization 0.73), 1.8 for
+// spacings of 1 : 2 : 0.5.  FP64: below 0.01, from leaving the mean out of the
+// transforms.
 // Component c of rows A and B is one complex line; its half rows go to W + c M.
 //
 // A line's T threads are lanes of one wavefront and every wavefront works
@@ -215,7 +222,13 @@ __device__ __forceinline__ void z_rhs_body(const Blk &bk, double2 *lds,
     const long ia = (act ? 2 * line : 0) * L; // row A; row B is L further
     double2 *wl = lds + wv * LPW * PITCH, *my = wl + lane / T * PITCH;
     double2 *const ltw = lds + z_rhs_lines<L, WG>();
-    [[maybe_unused]] C gx[E], gy[E], gz[E];
+    // what the sources are made from: FP64 the three gradients; FP32 the
+    // components themselves, rounded once from the FP64 gradients (products of
+    // gradients rounded to FP32 first: 4 to 7 % more error in the projected
+    // source of random fields, and the same time, 1277 and 1278 us for the
+    // right-hand side at 256^3)
+    constexpr int NG = sizeof(R) == 4 ? GW_NC : 3;
+    [[maybe_unused]] C g[NG][E];
     const double2 *const tw = ltw - L;
     if (!HELP || role == 0) {
     twiddles_to_lds_wave<L>(ltw, a.tw);
@@ -325,10 +338,22 @@ __device__ __forceinline__ void z_rhs_body(const Blk &bk, double2 *lds,
               v.dph.x, v.ps.x);
         point(i + L, p.y + dc, v.gx.y, v.gy.y, dz[s].y, v.lx.y + v.ly.y + lz[s].y,
               v.dph.y, v.ps.y);
-        if constexpr (GW) {
-            gx[s] = CT<C>::make((R)v.gx.x, (R)v.gx.y);
-            gy[s] = CT<C>::make((R)v.gy.x, (R)v.gy.y);
-            gz[s] = CT<C>::make((R)dz[s].x, (R)dz[s].y);
+        if constexpr (GW && sizeof(R) == 8) {
+            g[0][s] = v.gx;
+            g[1][s] = v.gy;
+            g[2][s] = dz[s];
+        } else if constexpr (GW) {
+            auto src = [&](auto kc) {
+                constexpr int K = decltype(kc)::value;
+                g[K][s] = CT<C>::make(
+                    (R)gw_source<K>(v.gx.x, v.gy.x, dz[s].x, a.ga.m),
+                    (R)gw_source<K>(v.gx.y, v.gy.y, dz[s].y, a.ga.m));
+            };
+            src(std::integral_constant<int, 0>{});
+            src(std::integral_constant<int, 1>{});
+            src(std::integral_constant<int, 2>{});
+            src(std::integral_constant<int, 3>{});
+            src(std::integral_constant<int, 4>{});
         }
     }
     srho = wave_reduce<OpSum>(srho);
@@ -340,23 +365,20 @@ __device__ __forceinline__ void z_rhs_body(const Blk &bk, double2 *lds,
     }
     }
     if constexpr (HELP) {
-        C *const g = reinterpret_cast<C *>(ltw + L) + lane;
+        static_assert(NG * sizeof(C) <= 3 * sizeof(double2), "see z_rhs_lds");
+        C *const sh = reinterpret_cast<C *>(ltw + L) + lane;
         if (role == 0) {
 #pragma unroll
-            for (int s = 0; s < E; ++s) {
-                g[64 * s] = gx[s];
-                g[64 * (E + s)] = gy[s];
-                g[64 * (2 * E + s)] = gz[s];
-            }
+            for (int q = 0; q < NG; ++q)
+#pragma unroll
+                for (int s = 0; s < E; ++s) sh[64 * (q * E + s)] = g[q][s];
         }
         lds_barrier();
         if (role != 0) {
 #pragma unroll
-            for (int s = 0; s < E; ++s) {
-                gx[s] = g[64 * s];
-                gy[s] = g[64 * (E + s)];
-                gz[s] = g[64 * (2 * E + s)];
-            }
+            for (int q = 0; q < NG; ++q)
+#pragma unroll
+                for (int s = 0; s < E; ++s) g[q][s] = sh[64 * (q * E + s)];
         }
     }
     if constexpr (GW) {
@@ -378,8 +400,12 @@ __device__ __forceinline__ void z_rhs_body(const Blk &bk, double2 *lds,
                 cmy, cmy, j, twc,
                 [&](int s, int) {
                     const int q = chain_slot<L, P>(s);
-                    return CT<C>::make(gw_source<K>(gx[q].x, gy[q].x, gz[q].x, a.ga.m),
-                                       gw_source<K>(gx[q].y, gy[q].y, gz[q].y, a.ga.m));
+                    if constexpr (sizeof(R) == 4)
+                        return g[K][q];
+                    else
+                        return CT<C>::make(
+                            gw_source<K>(g[0][q].x, g[1][q].x, g[2][q].x, a.ga.m),
+                            gw_source<K>(g[0][q].y, g[1][q].y, g[2][q].y, a.ga.m));
                 },
                 NoWrite());
             for (int idx = lane; idx < 2 * LPW * MZ; idx += 64) {

@@ -73,3 +73,29 @@ def test_fp32_gw_spectrum_per_bin(ih):
           np.array2string(rel, precision=2))
     assert live.sum() >= bins // 2
     assert rel.max() < 1e-4
+
+
+@pytest.mark.parametrize("n", [4, 8, 16, 32, 64])
+def test_fp32_products_are_rounded_once(ih, oracle_mod, n):
+    """One plane wave along each axis at a quarter of the sampling rate, with
+    gradients 0 and +-sqrt(7): every product is 0 or +-7 and everything after
+    it (transforms, projection on modes k (1, 1, 0)) is exact in FP32, so only
+    the rounding of the products themselves can show.  sqrt(7) rounded to FP32
+    first would give 7 (1 - 6.8e-8); the product rounded once from FP64 gives
+    7, and leaves the FP64 transforms' 2^-52 log2(n) per gradient, that is
+    1e-15, with a margin of 1000."""
+    shape, k = (n, n, n), n // 4
+    N = n ** 3
+    wave = np.sqrt(7.0) / k * np.cos(np.pi / 2 * np.arange(n))
+    y = make_state(shape, gw=False, amp=0.0, psi_amp=0.0)
+    y[:N] = 1.0 + (wave[:, None, None] + wave[None, :, None] + wave).ravel()
+    bounds = ((0.0, 2 * np.pi),) * 3
+    g = ih.Gpu(shape, bounds=bounds, gw=True, filt=False, bins=4, gw_fp32=True)
+    f, r = g.to_device(y), g.alloc(g.Ntot)
+    g.mk_rhs(f, r)
+    got = r.download()
+    g.close()
+    ref = oracle_mod.Oracle(*shape, bounds=bounds, gw=True, filt=False, bins=4).mk_rhs(y)
+    B = blocks(shape)
+    h = slice(B["dh1"].start, B["dh2"].stop)  # (dh2 is 0 on these modes)
+    assert rel_l2(got[h], ref[h]) < 1e-12
