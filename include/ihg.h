@@ -333,8 +333,10 @@ int ihg_init_gaussian(ihg_ctx *c, double *field, uint64_t seed,
 /* Autotuner of the strided y and x passes (no counterpart in the
  * reference): every candidate line plan, work-group size and tile order for
  * the y and the x line length is timed (three rounds of `reps` passes on the
- * context's work arrays, in the RHS's shape: four arrays, every realization
- * of an ensemble; each candidate's fastest round counts), and a candidate
+ * context's work arrays, in the RHS's shape: along y the filter's four arrays,
+ * along x the five components of the GW source, in FP32 where the source is;
+ * one array without the filter or without GW; every realization of an
+ * ensemble; each candidate's fastest round counts), and a candidate
  * replaces the default only when it is at least 3 % faster.  choice = {y, x}
  * candidate indices in use afterwards; ms (may be NULL) receives up to nms
  * average pass times, y candidates first.  Candidates differ in rounding

@@ -140,10 +140,12 @@ int fft_c2r(ihg_ctx *c, const double2 *in, double *out, double2 *work,
 }
 
 // Autotuner of the strided passes: every (plan, work-group) candidate of the
-// y and of the x line length is timed on the context's own work arrays, in
-// the shape the RHS uses most (four arrays, all realizations of an ensemble),
-// and the fastest is kept.  Results of different candidates differ only in
-// rounding.
+// y and of the x line length is timed on the context's own work arrays, with
+// the arrays the right-hand side gives that pass (all realizations of an
+// ensemble), and the fastest is kept: along y the filter's four, along x the
+// GW_NC components of the source, FP32 where they are; without the filter or
+// without GW the axis has one array, as in the transforms of an output call and
+// ihg_fft_*.  Results of different candidates differ only in rounding.
 template <int L>
 static int n_cands()
 {
@@ -189,8 +191,14 @@ int autotune(ihg_ctx *c, int reps, int out[2], float ms_out[16])
             for (int id = 0; id < ncand && id < 16 && !rc; ++id) {
                 slot = id;
                 auto pass = [&]() {
-                    return axis ? x_pass(c, c->W, -1, 4, c->M, nr, rr)
-                                : y_pass(c, c->W, -1, 4, c->M, nr, rr);
+                    if (!axis)
+                        return y_pass(c, c->W, -1, c->p.enable_filter ? 4 : 1,
+                                      c->M, nr, rr);
+                    if (c->p.enable_gw && c->p.gw_fp32)
+                        return x_pass_f32(c, reinterpret_cast<float2 *>(c->W), -1,
+                                          GW_NC, c->M, nr, 2 * rr);
+                    return x_pass(c, c->W, -1, c->p.enable_gw ? GW_NC : 1, c->M,
+                                  nr, rr);
                 };
                 rc = pass(); // warm-up
                 if (!rc) rc = hip_check(hipEventRecord(a, c->stream), "hipEventRecord");

@@ -133,6 +133,9 @@ struct ihg_ctx {
 
 namespace ihg {
 
+// components of the GW source that are transformed (see the z pass)
+constexpr int GW_NC = 5;
+
 struct ZShift;
 
 // FFT launchers (ihg_fft.hip)

@@ -100,7 +100,6 @@ struct FilterFac {
 // SIMD) against 8 (2 waves): 411 against 415 us at 256^3, 278 against 341 us
 // for 4 x 128^3, 5.1 against 9.3 us for one 32^3 grid without GW.
 // ---------------------------------------------------------------------------
-constexpr int GW_NC = 5;
 
 // The axis (0, 1, 2) whose diagonal product is subtracted from the others:
 // the one of the smallest Nyquist wave number, z where they are equal.
