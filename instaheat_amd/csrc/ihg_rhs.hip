@@ -396,9 +396,13 @@ static int rhs_gw_t(ihg_ctx *c, C *Wk, const C *tw, const double *f,
             if constexpr (L <= TT_WIDE_MAX) {
                 using TT = TTWide<L>;
                 const dim3 grid((unsigned)((ls.nlines + TT::B - 1) / TT::B), 1, nr);
+                // the RK4 epilogue where rk4_fusable has it
+                constexpr bool EP = std::is_same<C, double2>::value && L >= 16;
+                if (ep && !EP)
+                    return set_error("no RK4 epilogue for this TT pass");
                 return timed(c, F_TT_UPDATE_H, bytes, [&]() {
                     if (ep)
-                        hipLaunchKernelGGL((k_y_tt_wide<L, C, true>), grid,
+                        hipLaunchKernelGGL((k_y_tt_wide<L, C, EP>), grid,
                                            dim3(TT::WG), 0, c->stream, Wk, M, f,
                                            result, N, c->Next, c->Ntot, c->kg,
                                            c->dscal, ls, tw, e, rw,
