@@ -229,13 +229,17 @@ def test_autotuned_ensemble_rhs_matches_oracle(ih, E, oracle_mod):
 @pytest.mark.parametrize("shape,nreal,gw,fp32,flags", [
     ((16, 16, 16), 3, True, False, 1), ((32, 32, 32), 2, False, False, 0),
     ((128, 128, 128), 1, True, False, 0), ((16, 16, 16), 2, True, True, 1),
-    ((16, 256, 16), 2, True, False, 0)])
+    ((16, 256, 16), 2, True, False, 0), ((8, 128, 16), 3, True, False, 1),
+    ((16, 16, 16), 131, True, False, 0), ((32, 32, 32), 19, True, False, 1),
+    ((64, 64, 64), 3, True, False, 0), ((64, 64, 64), 1, False, False, 1)])
 def test_mk_rhs_rk4_equals_rhs_then_stage(ih, shape, nreal, gw, fp32, flags):
     """ihg_mk_rhs_rk4 (the stage or the final RK4 sum written by the kernels
     that write the slope) equals ihg_mk_rhs_ensemble followed by
     ihg_rk4_stage / ihg_rk4_final, bit for bit: 16^3 and 128^3 with GW
     (fused TT pass), 32^3 without GW, and the FP32 GW source and 256-point
-    y lines (no fused TT pass: the separate calls run)."""
+    y lines (no fused TT pass: the separate calls run).  The fused pass has
+    its components side by side up to 300000 modes (16^3 x 3, 8 x 128 x 16) and
+    in turn beyond (128^3, 16^3 x 131, 32^3 x 19, 64^3 x 3)."""
     L = ih.lib()
     p = ih.make_params(shape, BOX_CONFIG, 4.0, gw, True, 16, fp32)
     h = ctypes.c_void_p()
