@@ -102,11 +102,11 @@ def test_group_rhs_equals_per_context(ih, flags):
     n0 = L.ihg_group_launches(g)
     ih._check(L.ihg_group_mk_rhs(g, 0.0, _ptrs([c.f for c in ctxs]),
                                  _ptrs([c.r for c in ctxs]), flags))
-    # filter (5 passes) when any context filters, phi_hat for the others
-    # (2), fan-out with and without the kept spectrum, y, z c2r + rho, means,
-    # update, and the 3 GW passes
+    # the filter's z r2c, y, x round trip (of up to 64 points and of 128), y and
+    # z c2r; x and y derivatives and z pass of the contexts with GW and of those
+    # without; means, update; x pass and TT pass of the sources
     nl = L.ihg_group_launches(g) - n0
-    assert nl == (5 if flags else 0) + 2 + (2 if flags else 1) + 4 + 3, nl
+    assert nl == (6 if flags else 0) + 2 * 3 + 2 + 2, nl
     ih._check(L.ihg_sync(ctxs[0].ctx))
     got = [(c.download(c.r), c.download(c.f)) for c in ctxs]
     for c, (res, filt) in zip(ctxs, got):
@@ -118,6 +118,25 @@ def test_group_rhs_equals_per_context(ih, flags):
         assert np.array_equal(filt, c.download(f2))
         L.ihg_free(c.ctx, f2)
         L.ihg_free(c.ctx, r2)
+    L.ihg_group_destroy(g)
+    for c in ctxs:
+        c.close()
+
+
+@pytest.mark.parametrize("kinds,launches", [
+    (((32, True), (64, True)), 5 + 3 + 2 + 2),  # all GW, no 128-point grid
+    (((128, True),), 5 + 3 + 2 + 2),            # one context, its own round trip
+    (((16, False), (32, False)), 5 + 3 + 2)])   # no GW
+def test_group_launches_of_other_mixes(ih, kinds, launches):
+    L = ih.lib()
+    ctxs = [Ctx(ih, (n, n, n), 2, gw=gw, seed=10 * i) for i, (n, gw) in enumerate(kinds)]
+    g = _group(ih, ctxs)
+    print(f"grouped mk_rhs of {kinds}", flush=True)
+    n0 = L.ihg_group_launches(g)
+    ih._check(L.ihg_group_mk_rhs(g, 0.0, _ptrs([c.f for c in ctxs]),
+                                 _ptrs([c.r for c in ctxs]), 1))
+    assert L.ihg_group_launches(g) - n0 == launches
+    ih._check(L.ihg_sync(ctxs[0].ctx))
     L.ihg_group_destroy(g)
     for c in ctxs:
         c.close()

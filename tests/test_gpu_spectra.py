@@ -21,7 +21,8 @@ def test_spectra_at_tile_edges(oracle_mod, bins):
     o = oracle_mod.Oracle(*shape, bounds=BOX_CONFIG, gw=True, filt=True, bins=bins)
     fo = y.copy()
     o.mk_rhs(fo, filter=1, output=1, field=fo)
-    # a bin adds up to 2448 terms of one sign: rounding below 2448 * 2^-52
+    # a bin adds up to 8 * 16 * 17 = 2176 terms of one sign: rounding below
+    # 2176 * 2^-52
     for a, b in zip(got.reshape(4, bins), o.obs()[28:].reshape(4, bins)):
         assert rel_l2(a, b) < 1e-9
         assert np.all(np.isfinite(a))
