@@ -365,10 +365,20 @@ int rhs_core(ihg_ctx *c, double *f, double *result, int output, int filtered,
 // Whether the TT pass transforms the components side by side: up to about two
 // 64^3 grids.  Measured side by side and in turn: 7 x 16^3 6.2 and 13.3 us, 3
 // x 32^3 7.4 and 16.3, 64^3 (135 k modes) 12.0 and 13.1, 48 x 32^3 (836 k) 181
-// and 157, 128^3 (1.06 M) 71.8 and 68.9, 4 x 128^3 467 and 432 us.
+// and 157, 128^3 (1.06 M) 71.8 and 68.9, 4 x 128^3 467 and 432 us.  Near the
+// limit, whole right-hand sides: 17 x 32^3 (296 k) 61.0 and 64.4, 130 x 16^3
+// (300 k) 59.0 and 59.4, 512 x 64 x 16 (295 k) 78.1 and 81.3, 128 x 64 x 64 (270
+// k) 65.8 and 66.7, 3 x 64^3 (406 k) 75.6 and 72.5.
+// Lines of 128 points: a work-group takes 87 KB of LDS, one a CU, so the pass
+// must fit in one round: 32 x 128 x 32 (68 work-groups) 42.1 and 45.7, 3 x 64 x
+// 128 x 16 (216) 57.3 and 61.8, 32 x 128 x 128 (260) 75.0 and 69.3, 128 x 128 x
+// 32 (272) 70.4 and 65.4.
 static bool tt_wide(const ihg_ctx *c, int nr)
 {
-    return c->Ny <= TT_WIDE_MAX && c->M * nr < 300000;
+    if (c->Ny > TT_WIDE_MAX || c->M * nr >= 300000) return false;
+    constexpr int B = TTWide<128>::B;
+    const long lines = (long)c->Nx * c->Mz;
+    return c->Ny < 128 || (lines + B - 1) / B * nr <= NUM_CU;
 }
 
 // GW source pipeline on complex type C after the z pass: x pass, fused y
