@@ -200,7 +200,15 @@ ZShift filter_shift(const ihg_ctx *c, int nr)
 }
 
 // Work-group size of the derivative and z passes: single wavefronts while
-// 256 lanes a work-group would leave CUs idle.
+// 256 lanes a work-group would leave CUs idle.  Whole right-hand sides, 64 and
+// 256 lanes in one of the passes (in brackets its work-groups of 256 lanes):
+// derivatives 8 x 32^3 (256) 18.7 and 20.7 us, 64^3 (128) 19.5 and 20.8, 3 x
+// 64^3 (384) 33.4 and 33.3, 4 x 64^3 (512) 42.5 and 41.3, 128^3 (1024) 74.2 and
+// 70.7; z pass with GW 64^3 (128) 42.1 and 46.6, 128 x 64 x 128 (512) 104.6 and
+// 104.5, without GW 128^3 (1024) 73.0 and 70.2.  (In the z pass lines of 16 and
+// 32 points are faster with 64 lanes beyond the limit too: 48 x 32^3 (768) 139
+// and 153 us, 256 x 256 x 16 (512) 109 and 132; the rule makes no difference
+// between lengths.)
 static int small_wg(long blocks256) { return blocks256 < 512 ? 64 : 256; }
 
 template <int L, int WG>
@@ -313,7 +321,10 @@ int rhs_core(ihg_ctx *c, double *f, double *result, int output, int filtered,
     const double ep_blocks = !ep ? 0.0 : (ep->mode == RK4_FINAL ? 4.0 : 8.0);
     // one pair of points a thread on small grids (32^3 with the epilogue 5.1
     // against 5.9 us, 7 x 16^3 + 3 x 32^3 5.9 and 6.8), two on larger ones
-    // (64^3 6.2 against 7.0 us: the work-groups' sums count)
+    // (64^3 6.2 against 7.0 us: the work-groups' sums count).  Near the limit
+    // either choice is within 3 % of a right-hand side (131 to 197 k points:
+    // without the epilogue two pairs gain up to 0.4 us from 164 k on and lose
+    // up to 1 us at 131 k; with it one pair gains 0.2 to 1.7 us).
     const bool small = N * nr < 200000;
     const dim3 ugrid(nblocks(N, small ? RED_WG * 2 : RED_WG * 4, 65536), 1, nr);
     // One launch where the partial sums are few (64^3 has 512): 4.6 us against
