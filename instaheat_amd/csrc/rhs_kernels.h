@@ -368,16 +368,16 @@ __device__ __forceinline__ void z_rhs_body(const Blk &bk, double2 *lds,
         C *const sh = reinterpret_cast<C *>(ltw + L) + lane;
         if (role == 0) {
 #pragma unroll
-            for (int q = 0; q < NG; ++q)
+            for (int s = 0; s < E; ++s)
 #pragma unroll
-                for (int s = 0; s < E; ++s) sh[64 * (q * E + s)] = g[q][s];
+                for (int q = 0; q < NG; ++q) sh[64 * (q * E + s)] = g[q][s];
         }
         lds_barrier();
         if (role != 0) {
 #pragma unroll
-            for (int q = 0; q < NG; ++q)
+            for (int s = 0; s < E; ++s)
 #pragma unroll
-                for (int s = 0; s < E; ++s) g[q][s] = sh[64 * (q * E + s)];
+                for (int q = 0; q < NG; ++q) g[q][s] = sh[64 * (q * E + s)];
         }
     }
     if constexpr (GW) {
