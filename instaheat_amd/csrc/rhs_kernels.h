@@ -224,8 +224,8 @@ __device__ __forceinline__ void z_rhs_body(const Blk &bk, double2 *lds,
     // what the sources are made from: FP64 the three gradients; FP32 the
     // components themselves, rounded once from the FP64 gradients (products of
     // gradients rounded to FP32 first: 4 to 7 % more error in the projected
-    // source of random fields, and the same time, 1277 and 1278 us for the
-    // right-hand side at 256^3)
+    // source of random fields; this pass 391 us then and 394 now, the
+    // right-hand side 1277 and 1278 at 256^3)
     constexpr int NG = sizeof(R) == 4 ? GW_NC : 3;
     [[maybe_unused]] C g[NG][E];
     const double2 *const tw = ltw - L;
